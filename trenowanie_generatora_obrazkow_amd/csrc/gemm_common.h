@@ -93,6 +93,31 @@ __device__ __forceinline__ void buf2lds(uint32_t voff, i32x4 rsrc, uint32_t soff
                :: "s"(m0), "v"(voff), "s"(rsrc), "s"(soff) : "memory", "m0");
 }
 
+// The same copy for the branch-free inner iterations, to LDS address lds32 + OFF (OFF a compile-time offset).  There the
+// issue slots are what counts: one wave per SIMD issues an instruction about every 4 cycles and an MFMA occupies the
+// matrix core for 32, so more than seven instructions between two MFMAs leave it idle, and a copy in buf2lds' form (the
+// generic pointer's null test, M0, five wait states) takes nine.  This form takes three: the scalar operands are used as
+// they are and only M0's own wait state is kept.  It relies on no VALU instruction writing one of its scalar operands in
+// the five wait states before it; the compiler cannot see that, so a test checks the built code for it.
+template <int OFF>
+__device__ __forceinline__ void buf2lds_inner(uint32_t voff, const i32x4& rsrc, uint32_t soff, uint32_t lds32) {
+  asm volatile("s_add_u32 m0, %0, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+               :: "s"(lds32), "v"(voff), "s"(rsrc), "s"(soff), "i"(OFF) : "memory", "m0", "scc");
+}
+
+__device__ __forceinline__ uint32_t lds_addr(const char* p) {
+  return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)p;
+}
+
+// f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>)
+template <int N, class F, int I = 0>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for<N, F, I + 1>(static_cast<F&&>(f));
+  }
+}
+
 // K-major operand: ROWS rows x 32 k per slice; ROWS/16 copy instructions per slice (each 16 rows x 64 bytes),
 // spread over the workgroup's waves.
 template <int ROWS, int NWAVES>
@@ -123,9 +148,11 @@ struct KTile {
     const uint32_t vo = (k0 + kBK <= K || k0 + chunk[i] * 8 < K) ? voff[i] : kOOB;
     buf2lds(vo, rsrc, (uint32_t)k0 * kmul, lds_tile + (wave * PER_WAVE + i) * 1024);
   }
-  // the same for a slice known to lie inside K (no tail test)
-  __device__ __forceinline__ void issue_one_full(char* lds_tile, int wave, int i, int k0) const {
-    buf2lds(voff[i], rsrc, (uint32_t)k0 * kmul, lds_tile + (wave * PER_WAVE + i) * 1024);
+  // the same for a slice known to lie inside K: soff = soff_of(k0), part32 = LDS address of the wave's part of the tile
+  __device__ __forceinline__ uint32_t soff_of(int k0) const { return (uint32_t)k0 * kmul; }
+  template <int I>
+  __device__ __forceinline__ void issue_inner(uint32_t part32, uint32_t soff) const {
+    buf2lds_inner<I * 1024>(voff[I], rsrc, soff, part32);
   }
   // Lane part of a fragment read address: row w32*32 + lane%32, k-chunk lane/32 (ks = 0), swizzled.  The
   // swizzle of row grp64 + w32*32 + lane%32 is that of lane%32, and chunk 2 + c stored at (2 + c) ^ s = (c ^ s) ^ 2,
@@ -168,8 +195,11 @@ struct MNTile {
     const uint32_t vo = (k0 + kBK <= Kvalid || k0 + krow[i] < Kvalid) ? voff[i] : kOOB;
     buf2lds(vo, rsrc, (uint32_t)k0 * kstep, lds_tile + (wave * PER_WAVE + i) * 1024);
   }
-  __device__ __forceinline__ void issue_one_full(char* lds_tile, int wave, int i, int k0) const {
-    buf2lds(voff[i], rsrc, (uint32_t)k0 * kstep, lds_tile + (wave * PER_WAVE + i) * 1024);
+  // the same for a slice known to lie inside K: soff = soff_of(k0), part32 = LDS address of the wave's part of the tile
+  __device__ __forceinline__ uint32_t soff_of(int k0) const { return (uint32_t)k0 * kstep; }
+  template <int I>
+  __device__ __forceinline__ void issue_inner(uint32_t part32, uint32_t soff) const {
+    buf2lds_inner<I * 1024>(voff[I], rsrc, soff, part32);
   }
   // lane l of instruction (wave w, i): k-row (w*PER_WAVE + i)*KPI + l / CPR, physical chunk l % CPR
   __device__ __forceinline__ static void slot(int wave, int lane, int i, int& k, int& col) {
@@ -237,8 +267,11 @@ struct MNTile8 {
     const uint32_t vo = (k0 + kBK <= Kvalid || k0 + krow[i] < Kvalid) ? voff[i] : kOOB;
     buf2lds(vo, rsrc, (uint32_t)k0 * kstep, lds_tile + (wave * PER_WAVE + i) * 1024);
   }
-  __device__ __forceinline__ void issue_one_full(char* lds_tile, int wave, int i, int k0) const {
-    buf2lds(voff[i], rsrc, (uint32_t)k0 * kstep, lds_tile + (wave * PER_WAVE + i) * 1024);
+  // the same for a slice known to lie inside K: soff = soff_of(k0), part32 = LDS address of the wave's part of the tile
+  __device__ __forceinline__ uint32_t soff_of(int k0) const { return (uint32_t)k0 * kstep; }
+  template <int I>
+  __device__ __forceinline__ void issue_inner(uint32_t part32, uint32_t soff) const {
+    buf2lds_inner<I * 1024>(voff[I], rsrc, soff, part32);
   }
   // lane l of instruction (wave w, i): k-row (w*PER_WAVE + i)*KPI + l / CPR, physical chunk l % CPR; col = the first
   // logical column the slot holds
@@ -255,24 +288,33 @@ struct MNTile8 {
     const int h = (lane >> 4) & 1;
     return kr * ROWS + 16 * FN * ((2 * w32 + h) ^ (kr & 3)) + 8 * (lane & 1);
   }
-  // fragment b (columns b*FSN + 32 w32 + 0..31) x 16 k (ks*16 + ...), converted exactly to bf16 (fp16 with F16)
-  __device__ __forceinline__ static bf16x8 frag(const char* lds_tile, int grp64, int loff, int ks) {
-    typedef int i32x2 __attribute__((ext_vector_type(2)));
-    typedef __attribute__((address_space(3))) i32x2 lds_i32x2;
-    const int b = grp64 / 64;
-    const i32x2 v = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_i32x2*)(lds_tile + loff + ks * 16 * ROWS + 16 * b));
-    // signed bytes -> exact floats (|q| <= 128 has at most 8 significant bits) -> bf16; each byte converts in one
-    // instruction (a sign-extending byte select on the int -> float conversion)
-    const uint32_t lo = (uint32_t)v[0], hi = (uint32_t)v[1];
-    float f[8];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      f[j] = (float)(int8_t)(lo >> (8 * j));
-      f[4 + j] = (float)(int8_t)(hi >> (8 * j));
+  typedef int Raw __attribute__((ext_vector_type(2)));  // a lane's 8 bytes of a fragment
+  // fragment b (columns b*FSN + 32 w32 + 0..31) x 16 k (ks*16 + ...) as bytes
+  __device__ __forceinline__ static Raw frag_raw(const char* lds_tile, int grp64, int loff, int ks) {
+    typedef __attribute__((address_space(3))) Raw lds_raw;
+    return __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_raw*)(lds_tile + loff + ks * 16 * ROWS + 16 * (grp64 / 64)));
+  }
+  // its elements 2 P and 2 P + 1 (P = 0..3) converted exactly and packed.  bf16: signed bytes -> exact floats (|q| <= 128
+  // has at most 8 significant bits) -> bf16, one instruction per byte (a sign-extending byte select on the int -> float
+  // conversion) and one per pair.  fp16: the byte q + 128 under the exponent byte of 1024 is the fp16 number 1152 + q, and
+  // subtracting 1152 is exact: a byte permute and a packed subtraction per pair.
+  template <int P>
+  __device__ __forceinline__ static uint32_t convert(Raw v) {
+    const uint32_t w = (uint32_t)v[P / 2];
+    constexpr int b = 2 * (P & 1);  // the pair's first byte
+    if constexpr (F16) {
+      typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+      const uint32_t t = __builtin_amdgcn_perm(0x64646464u, w ^ 0x80808080u, 0x04000400u | b | ((b + 1) << 16));
+      const f16x2 r = __builtin_bit_cast(f16x2, t) - f16x2{(_Float16)1152.0f, (_Float16)1152.0f};
+      return __builtin_bit_cast(uint32_t, r);
+    } else {
+      return Elt<F16>::pack2((float)(int8_t)(w >> (8 * b)), (float)(int8_t)(w >> (8 * b + 8)));
     }
+  }
+  __device__ __forceinline__ static bf16x8 frag(const char* lds_tile, int grp64, int loff, int ks) {
+    const Raw v = frag_raw(lds_tile, grp64, loff, ks);
     typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-    using X = Elt<F16>;
-    const u32x4 w = {X::pack2(f[0], f[1]), X::pack2(f[2], f[3]), X::pack2(f[4], f[5]), X::pack2(f[6], f[7])};
+    const u32x4 w = {convert<0>(v), convert<1>(v), convert<2>(v), convert<3>(v)};
     return __builtin_bit_cast(bf16x8, w);
   }
 };
