@@ -1,0 +1,69 @@
+"""The few-rows GEMM kernel (csrc/gemm_few.h) against the persistent kernel, which the oracle tests pin: both run the same
+MFMAs in the same k order and round at the same places, so the results are equal bit for bit.  Sizes sit at the edges of
+its tiles (32, 64 and 128 rows; 128 and 256 columns), with empty experts, experts of several m-tiles, k-slices fewer than
+the ring holds, and ragged K and N."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# rows per expert; (columns, K): chosen so that the rule takes the tile named (E, M and the columns decide)
+EDGE32 = [0, 1, 31, 32, 33, 0, 64, 5, 97]
+CASES = {
+    "32x128-one-expert": ([40], 136, 72),
+    "32x128-edges": (EDGE32, 264, 1000),
+    "32x128-short-k": (EDGE32, 1024, 24),
+    "32x128-few-rows-many-experts": ([0] * 100 + [1, 0, 2] + [0] * 153, 512, 544),
+    "64x256-edges": ([0, 1, 63, 64, 65, 2, 0, 130] * 8, 520, 544),
+    "64x256-skew": ([600] + [3] * 60 + [0, 0, 0], 776, 40),
+    "64x256-256-experts": ([4, 0, 9, 7] * 64, 272, 96),
+    "128x256-edges": ([127, 128, 129, 0, 1, 64, 65, 200] * 4, 1304, 264),
+    "128x256-skew": ([1100] + [50] * 30 + [0], 1544, 64),
+    "257-experts": ([2, 1, 0] * 85 + [3, 1], 528, 136),  # past the kernel's expert limit: the persistent one
+}
+
+
+def _inputs(counts, dt, K, gen):
+    E, M = len(counts), sum(counts)
+    T = max(M // 2, 1)
+    c = torch.tensor(counts, dtype=torch.int32)
+    x = torch.randn(T, K, generator=gen).to(dt)
+    a_idx = torch.randint(0, T, (M,), generator=gen).int()
+    y_idx = torch.randperm(M, generator=gen).int()
+    return E, M, c.cuda(), x.cuda(), a_idx.cuda(), y_idx.cuda(), torch.rand(M, generator=gen).to(dt).cuda()
+
+
+def _weights(E, K, N, dt, quant, gen):
+    if not quant:
+        return (torch.randn(E, K, N, generator=gen) * K ** -0.5).to(dt).cuda(), None
+    q = torch.randint(-128, 128, (E, K, N), generator=gen, dtype=torch.int8).cuda()
+    s = (torch.rand(E, N, generator=gen) * 0.02 + 1e-3).to(torch.bfloat16 if quant == "bf16" else torch.float32)
+    return q, s.cuda()
+
+
+@pytest.mark.parametrize("dt,quant", [(torch.bfloat16, None), (torch.float16, None), (torch.bfloat16, "bf16"),
+                                      (torch.float16, "fp32")])
+@pytest.mark.parametrize("case", CASES)
+def test_bit_identical_to_persistent(case, dt, quant, monkeypatch):
+    from trenowanie_generatora_obrazkow_amd import ops
+    counts, N, K = CASES[case]
+    N = -(-N // 16) * 16 if quant else N
+    print(f"few rows {case} {dt} quant={quant}", flush=True)
+    gen = torch.Generator().manual_seed(len(case) + K)
+    E, M, c, x, a_idx, y_idx, scale = _inputs(counts, dt, K, gen)
+    w, ws = _weights(E, K, N, dt, quant, gen)
+    wgu, gs = _weights(E, K, 2 * N, dt, quant, gen)
+    xs = x[a_idx.long()].contiguous()
+
+    def run():
+        return [ops.grouped_mm(x, w, c, M, a_idx=a_idx, y_idx=y_idx, scale=scale, w_scale=ws),
+                ops.grouped_mm(xs, w, c.long(), M, scale=scale.float(), w_scale=ws),
+                ops.down_scatter(xs, w, c, M, scale, y_idx, wd_s=ws)[0],
+                ops.gate_up_swiglu(x, wgu, c, M, a_idx=a_idx, wgu_s=gs)[0],
+                ops.gate_up_swiglu(xs, wgu, c, M, wgu_s=gs)[0]]
+
+    got = run()
+    monkeypatch.setenv("HMOE_GEMM_TILE", "S")
+    want = run()
+    for i, (a, b) in enumerate(zip(got, want)):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16)), f"{case}: call {i}"

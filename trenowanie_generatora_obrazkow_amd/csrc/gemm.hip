@@ -20,6 +20,7 @@
 // MFMA roles: the N-side tile feeds the MFMA "A" operand and the M-side tile the "B" operand, so each lane's
 // accumulator holds one output row and 4 consecutive output columns per group -> 8-byte bf16 / 16-byte fp32 stores.
 #include "gemm_common.h"
+#include "gemm_few.h"
 
 #include <algorithm>
 #include <atomic>
@@ -1103,9 +1104,77 @@ static int launch_mgroup(const GemmParams& p, int64_t ncols, hipStream_t s) {
   return launch<CfgS, MODE, A_MN, B_MN, EPI, A_BLK, F16>(p, mgroup_tiles<CfgS, EPI>(p.M, p.E, ncols), s);
 }
 
+template <class C, int EPI, bool F16>
+static int launch_few_tile(const GemmParams& p, int64_t ncols, hipStream_t s) {
+  auto kern = few_rows_gemm_kernel<C, EPI, F16>;
+  static std::atomic<bool> attr_set[64];  // per device, as in launch()
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return HMOE_ERR_DEVICE;
+  if (!attr_set[dev].load(std::memory_order_acquire)) {
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                            C::LDS_BYTES) != hipSuccess)
+      return HMOE_ERR_LAUNCH;
+    attr_set[dev].store(true, std::memory_order_release);
+  }
+  const int64_t bn = EPI == EPI_SWIGLU ? C::BN / 2 : C::BN;
+  // the experts' first m-tiles, then at most M / BM further ones, both in eights (one per XCD)
+  const int64_t nb_n = (ncols + bn - 1) / bn, mt = (p.E + 7) / 8 * 8 + (p.M / C::BM + 7) / 8 * 8;
+  hipLaunchKernelGGL(kern, dim3((unsigned)(mt * nb_n)), dim3(C::NT), C::LDS_BYTES, s, p, (int)nb_n);
+  HMOE_CHECK_LAUNCH();
+  return HMOE_OK;
+}
+
+// The few-rows kernel (gemm_few.h) or the persistent one.  Measured on MI355X over 8 layers (d 256-2048, h 320-4096, 1-128
+// experts, bf16, fp16 and int8 weights), 2 to 256 routed rows per expert, gate/up and down, every tile against the
+// persistent kernel's choice in one process; us, persistent -> few:
+//   d 2048, h 320, 128 int8 experts: 4 rows per expert 59.5 -> 31.7 (gate/up) and 34.4 -> 24.3 (down), 32 rows 60 -> 37
+//   and 35.5 -> 28.5, 96 rows 69.9 -> 57.7 and 41.9 -> 42.5; d 2048, h 1408, 64 int8 experts: 2 rows 92.8 -> 59.7 and
+//   48 -> 32, 96 rows 129 -> 109 and 59.7 -> 50.7; d 1536, h 1024, 60 fp16 experts: 48 rows 79.1 -> 75.5 and 45 -> 36.8,
+//   96 rows 88.5 -> 83.4 and 50.2 -> 44.6; d 256, h 512, 8 experts: 128 rows 8.8 -> 7.3 and 10.1 -> 7.8.
+// Tiles: 64 rows x 256 columns up to 52 rows per expert (above, most experts need a second tile, which reads the weights
+// again), then 128 x 256, or 64 x 256 where those leave too few workgroups.  Where even a third of a workgroup per CU is
+// not reached, 32 x 128, while these give no more than 3/4 of a workgroup per CU (1.5 with K up to 512: the launch is
+// then a handful of latencies long).  Above 144 (int8) or 112 rows per expert the products bound the launch and the
+// persistent kernel's 256-row tiles win (128 rows: fp16 gate/up 92.8 against 99.8, int8 154.5 against 129.7; 192 rows:
+// int8 176 against 204).
+enum FewTile { FEW_NONE, FEW_32x128, FEW_64x256, FEW_128x256 };
+template <int EPI>
+static FewTile pick_few(int64_t M, int64_t E, int64_t ncols, int64_t K, bool int8) {
+  if (E > kFewMaxE || M > kFewMaxM || env_force()) return FEW_NONE;
+  const int64_t cus = cu_count(), act = std::min(E, M);  // (at most M experts have rows)
+  auto tiles = [&](int64_t bm, int64_t bn) {
+    const int64_t cols = EPI == EPI_SWIGLU ? bn / 2 : bn;
+    return (act + M / bm) * ((ncols + cols - 1) / cols);
+  };
+  const int64_t ta = tiles(32, 128);
+  if (ta * 4 <= cus * 3 || (ta * 2 <= cus * 3 && K <= 512)) return FEW_32x128;
+  if (M > E * (int8 ? 144 : 112)) return FEW_NONE;
+  if (M > E * 52 && tiles(128, 256) >= cus) return FEW_128x256;
+  return tiles(64, 256) * 8 >= cus * 3 ? FEW_64x256 : FEW_NONE;
+}
+
+// launches the few-rows kernel if the rule picks it: *done, and the launch's status
+template <int EPI, bool F16, int BE>
+static int launch_few(const GemmParams& p, int64_t ncols, hipStream_t s, bool* done) {
+  // (a [g | u] or unscaled copy is the persistent kernel's)
+  const FewTile t = p.aux ? FEW_NONE : pick_few<EPI>(p.M, p.E, ncols, p.K, BE == 1);
+  *done = t != FEW_NONE;
+  switch (t) {
+    case FEW_32x128: return launch_few_tile<FewCfg<1, 2, 4, BE>, EPI, F16>(p, ncols, s);
+    case FEW_64x256: return launch_few_tile<FewCfg<2, 4, 3, BE>, EPI, F16>(p, ncols, s);
+    case FEW_128x256: return launch_few_tile<FewCfg<4, 4, 3, BE>, EPI, F16>(p, ncols, s);
+    default: return HMOE_OK;
+  }
+}
+
 // the bf16 (f16 = false) or fp16 form of a forward launch
 template <int EPI, bool A_BLK = false>
 static int launch_fwd(const GemmParams& p, int64_t ncols, bool f16, hipStream_t s) {
+  if constexpr (!A_BLK) {
+    bool done;
+    const int rc = f16 ? launch_few<EPI, true, 2>(p, ncols, s, &done) : launch_few<EPI, false, 2>(p, ncols, s, &done);
+    if (done) return rc;
+  }
   return f16 ? launch_mgroup<MGROUP, false, true, EPI, A_BLK, true>(p, ncols, s)
              : launch_mgroup<MGROUP, false, true, EPI, A_BLK, false>(p, ncols, s);
 }
@@ -1113,6 +1182,9 @@ static int launch_fwd(const GemmParams& p, int64_t ncols, bool f16, hipStream_t 
 // int8 weights: the int8 tile configurations
 template <int EPI, bool F16 = false>
 static int launch_mgroup_i8_t(const GemmParams& p, int64_t ncols, hipStream_t s) {
+  bool done;
+  const int rc = launch_few<EPI, F16, 1>(p, ncols, s, &done);
+  if (done) return rc;
   const int64_t tl = mgroup_tiles<CfgL8, EPI>(p.M, p.E, ncols);
   bool large = pick_large_mgroup<EPI>(tl, ncols, p.K, true);
   // gate/up with many experts (E >= 128): the tile bound counts a partial tile per expert, and below 3.25 large

@@ -1,0 +1,317 @@
+// Grouped GEMM for few rows per expert (prompts and small batches over many experts), forward projections with the
+// weights N-contiguous: the launch streams every weight once and is bound by how many of their bytes are in flight.
+//
+// The persistent kernel (gemm.hip) gives a CU one 256x256 tile or two 128x128 ones: most of its ring and copy slots hold
+// rows of A, of which there are few here, and each tile's prologue (counts, expert scan, row ids), short main loop and
+// epilogue follow one another.  Here a workgroup is one tile of 32 FR rows x 64 columns per wave (SwiGLU: half of them gate
+// columns, half the matching up columns) and a CU holds two to six of them, so one fills its ring while another multiplies
+// or stores; what a tile's epilogue reads (row scatter index, routing weight, column scales) is loaded ahead of its first
+// copy.  Four waves side by side give 256-byte (16-bit) or 128-byte (int8) pieces of a gate row: half-line pieces measured
+// up to 25% slower.  A shallow ring and more workgroups per CU beat a deep ring (d 2048, h 320, 128 int8 experts, 4 rows
+// per expert, down: rings of 12, 8, 6, 5 and 4 slices with 32 rows 50.6, 36.4, 28.9, 23.8 and 22.7 us).
+// The ring is NS slices of 32 k deep with NS - 1 in flight; every iteration issues a whole slice (past K: copies outside
+// the range, which move nothing), so the wait counts are constants.
+//
+// The products and their order in k are those of the persistent kernel (the same 32x32x16 MFMAs in k order from zero), and
+// so are the roundings of the epilogues: the results are bit-identical.
+//
+// Measured (GB/s of weights read once): 24 tokens, top-6 of 64 int8 experts, d 2048, h 1408: gate/up 90 -> 59 us (5650),
+// down 47.5 -> 30.8 (5400); 64 tokens, top-8 of 128, h 320: 58 -> 31 (5400) and 34 -> 23.6 (3560).
+#pragma once
+#include "gemm_common.h"
+
+namespace hmoe {
+
+template <int FR_, int W_, int NS_, int BE_>
+struct FewCfg {
+  static constexpr int FR = FR_, NWAVES = W_, NS = NS_, BE = BE_;  // row fragments, waves, ring slices, bytes per weight
+  static constexpr int BM = 32 * FR, BN = 64 * NWAVES, NT = 64 * NWAVES;
+  static constexpr int A_BYTES = BM * kBK * 2, B_BYTES = BN * kBK * BE, STAGE_BYTES = A_BYTES + B_BYTES;
+  static constexpr int LDS_BYTES = NS * STAGE_BYTES;
+};
+constexpr int kFewMaxE = 256;           // experts: four per lane in the scan of the counts
+constexpr int64_t kFewMaxM = 1 << 20;  // rows (32-bit row arithmetic)
+
+template <class C, int EPI, bool F16>
+__global__ __launch_bounds__(C::NT, 2) void few_rows_gemm_kernel(GemmParams p, int nb_n) {
+  static_assert(EPI == EPI_STORE || EPI == EPI_SWIGLU, "forward epilogues");
+  using X = Elt<F16>;
+  using TA = KTile<C::BM, C::NWAVES>;
+  using TB = typename TileSel<true, C::BN, C::NWAVES, C::BE, C::NWAVES, F16>::type;
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int E = p.E;
+
+  // ---- the workgroup's tile: m-tiles [0, E) are the first one of their expert, the others the experts' further ones in
+  // order (at most M / BM of them).  Each wave scans the counts by itself, up to four experts per lane.
+  // Workgroups go to the 8 XCDs in turn: all n-tiles of an m-tile take ids of one XCD, next to each other, so that the
+  // weight lines two of them share (64-byte halves with int8 gate / up columns) are fetched into its L2 once.
+  const int q = (int)blockIdx.x >> 3;
+  int mt = (q / nb_n) * 8 + ((int)blockIdx.x & 7);
+  const int nb = q % nb_n;
+  const int Ep = (E + 7) & ~7;
+  if (mt >= E && mt < Ep) return;
+  if (mt >= Ep) mt -= Ep - E;
+  const int per = (E + 63) / 64;
+  int cnt[4], rs = 0, ov = 0;  // counts of the lane's experts; their rows, and their m-tiles after the first
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int e = lane * per + i;
+    int64_t c = 0;
+    if (i < per && e < E) c = read_count(p.counts, p.counts64, e);
+    cnt[i] = (int)(c < 0 ? 0 : (c > p.M ? p.M : c));
+    rs = (int)min((int64_t)rs + cnt[i], p.M);  // (garbage counts must not overflow)
+    ov += cnt[i] > 0 ? (cnt[i] - 1) / C::BM : 0;
+  }
+  int irs = rs, iov = ov;
+#pragma unroll
+  for (int s = 1; s < 64; s <<= 1) {
+    const int a = __shfl_up(irs, s, 64), b = __shfl_up(iov, s, 64);
+    if (lane >= s) {
+      irs = (int)min((int64_t)irs + a, p.M);
+      iov += b;
+    }
+  }
+  int e, j = 0;  // expert and its m-tile
+  if (mt < E) {
+    e = mt;
+  } else {
+    const int want = mt - E;
+    const uint64_t owner = __ballot(iov > want);  // lanes are in expert order: the first one holds the tile
+    if (owner == 0) return;                       // (the same in both waves)
+    const int ol = __builtin_ctzll(owner);
+    int left = want - __shfl(iov - ov, ol, 64);
+    e = ol * per;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int c = __shfl(cnt[i], ol, 64);
+      const int t = c > 0 ? (c - 1) / C::BM : 0;
+      if (j == 0) {
+        if (left < t) {
+          j = left + 1;
+          e = ol * per + i;
+        } else {
+          left -= t;
+        }
+      }
+    }
+  }
+  int row0 = __shfl(irs - rs, e / per, 64), rows = 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int c = __shfl(cnt[i], e / per, 64);
+    if (i < e % per) row0 += c;
+    if (i == e % per) rows = c;
+  }
+  row0 += j * C::BM;
+  e = __builtin_amdgcn_readfirstlane(e);
+  row0 = __builtin_amdgcn_readfirstlane(row0);
+  const int row_end = __builtin_amdgcn_readfirstlane((int)min((int64_t)row0 + min(rows - j * C::BM, C::BM), p.M));
+  if (row0 >= row_end) return;
+  const int n0 = nb * (EPI == EPI_SWIGLU ? C::BN / 2 : C::BN);
+
+  // ---- copy sources ----
+  TA ta;
+  TB tb;
+  ta.K = p.K;
+  ta.rsrc = make_rsrc(p.a_idx ? p.A : p.A + (int64_t)row0 * p.lda);
+#pragma unroll
+  for (int i = 0; i < TA::PER_WAVE; ++i) {
+    const int rr = TA::row_of(wave, lane, i);
+    const int c = (lane & 3) ^ swz_k(rr);
+    ta.voff[i] = kOOB;
+    if (row0 + rr < row_end) {
+      const int64_t src = p.a_idx ? (int64_t)p.a_idx[row0 + rr] : (int64_t)rr;
+      ta.voff[i] = (uint32_t)(src * p.lda * 2 + c * 16);
+    }
+    ta.chunk[i] = c;
+  }
+  tb.rsrc = make_rsrc(static_cast<const char*>(p.B) + (int64_t)e * p.strideBe * C::BE);
+  tb.kstep = (uint32_t)(p.ldb * C::BE);
+  tb.Kvalid = p.K;
+#pragma unroll
+  for (int i = 0; i < TB::PER_WAVE; ++i) {
+    int k, nn;
+    TB::slot(wave, lane, i, k, nn);
+    int col = n0 + nn;
+    bool ok = col < p.N;
+    if (EPI == EPI_SWIGLU) {  // tile columns [0, 64) gate, [64, 128) the matching up
+      const int ac = n0 + nn % (C::BN / 2);
+      col = nn / (C::BN / 2) * p.h + ac;
+      ok = ac < p.N;
+    }
+    tb.krow[i] = k;
+    tb.voff[i] = ok ? (uint32_t)(((int64_t)k * p.ldb + col) * C::BE) : kOOB;
+  }
+
+  // ---- epilogue inputs, loaded ahead of the copies: the lane's rows' scatter index and scale (row a*32 + lane%32), and
+  // with int8 weights its columns' scales (column halves b, groups g; a lane holds 4 consecutive columns per group) ----
+  [[maybe_unused]] int yr[C::FR];
+  [[maybe_unused]] float sc[C::FR];
+  if constexpr (EPI == EPI_STORE) {
+#pragma unroll
+    for (int a = 0; a < C::FR; ++a) {
+      const int row = row0 + a * 32 + (lane & 31);
+      yr[a] = row;
+      sc[a] = 1.0f;  // the product is then exact
+      if (row < row_end) {
+        if (p.y_idx) yr[a] = p.y_idx[row];
+        if (p.scale)
+          sc[a] = p.scale_f32 ? static_cast<const float*>(p.scale)[row]
+                              : X::one(static_cast<const uint16_t*>(p.scale)[row]);
+      }
+    }
+  }
+  [[maybe_unused]] float cs[2][4][4];
+  if constexpr (C::BE == 1) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int lc = wave * 32 + 8 * g + 4 * (lane >> 5);
+        const int col = EPI == EPI_SWIGLU ? b * p.h + n0 + lc : n0 + C::BN / 2 * b + lc;
+        const bool ok = (EPI == EPI_SWIGLU ? n0 + lc : col) < p.N;
+        const int64_t at = (int64_t)e * p.ldws + col;
+        float* v = cs[b][g];
+        if (p.w_scale_f32) {
+          const float4 w = ok ? *reinterpret_cast<const float4*>(static_cast<const float*>(p.w_scale) + at)
+                              : make_float4(0.f, 0.f, 0.f, 0.f);
+          v[0] = w.x; v[1] = w.y; v[2] = w.z; v[3] = w.w;
+        } else {
+          const uint2 w = ok ? *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(p.w_scale) + at)
+                             : make_uint2(0u, 0u);
+          v[0] = bf_lo(w.x); v[1] = bf_hi(w.x); v[2] = bf_lo(w.y); v[3] = bf_hi(w.y);
+        }
+      }
+  }
+
+  // ---- main loop ----
+  constexpr int LOADS = TA::PER_WAVE + TB::PER_WAVE;
+  const int nk = (p.K + kBK - 1) / kBK;
+  auto issue = [&](int s) {  // slice s into its slot; past the last slice copies that move nothing
+    char* slot = smem + (s % C::NS) * C::STAGE_BYTES;
+    if (s < nk) {
+      ta.issue(slot, wave, lane, s * kBK);
+      tb.issue(slot + C::A_BYTES, wave, lane, s * kBK);
+    } else {
+#pragma unroll
+      for (int i = 0; i < LOADS; ++i) buf2lds(kOOB, tb.rsrc, 0u, slot + (wave * LOADS + i) * 1024);
+    }
+  };
+  const int loff_a = TA::lane_off(0, lane), loff_b = TB::lane_off(wave & 1, lane);
+  f32x16 acc[C::FR][2];
+#pragma unroll
+  for (int a = 0; a < C::FR; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.0f;
+  auto main_loop = [&](auto fe_tag) {  // FE: row fragments holding rows (of FR)
+    constexpr int FE = decltype(fe_tag)::value;
+#pragma unroll
+    for (int s = 0; s < C::NS - 1; ++s) issue(s);
+    uint32_t cons = 0, fill = (C::NS - 1) * C::STAGE_BYTES;  // ring offsets: the slot filled is that of slice kt - 1
+    const uint32_t pa = lds_addr(smem) + wave * (TA::PER_WAVE * 1024);
+    const uint32_t pb = lds_addr(smem) + C::A_BYTES + wave * (TB::PER_WAVE * 1024);
+    auto iter = [&](int kt, auto fast_tag) {
+      wait_vm<(C::NS - 2) * LOADS>();  // this wave's copies of slice kt have landed
+      lds_barrier();                   // and the others'; all have read slice kt - 1, whose slot is filled next
+      if constexpr (decltype(fast_tag)::value) {
+        const int k0 = (kt + C::NS - 1) * kBK;
+        const uint32_t sa = ta.soff_of(k0), sb = tb.soff_of(k0);
+        static_for<TA::PER_WAVE>([&](auto l) { ta.template issue_inner<decltype(l)::value>(pa + fill, sa); });
+        static_for<TB::PER_WAVE>([&](auto l) { tb.template issue_inner<decltype(l)::value>(pb + fill, sb); });
+      } else {
+        issue(kt + C::NS - 1);
+      }
+      const char* slot = smem + cons;
+      fill = cons;
+      cons += C::STAGE_BYTES;
+      if (cons == C::LDS_BYTES) cons = 0;
+      bf16x8 xa[2][FE], wb[2][2];
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b) wb[ks][b] = TB::frag(slot + C::A_BYTES, b * (C::BN / 2) + 64 * (wave >> 1), loff_b, ks);
+#pragma unroll
+        for (int a = 0; a < FE; ++a) xa[ks][a] = TA::frag(slot, 32 * a, loff_a, ks);
+      }
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int a = 0; a < FE; ++a)
+#pragma unroll
+          for (int b = 0; b < 2; ++b) acc[a][b] = mfma16<F16>(wb[ks][b], xa[ks][a], acc[a][b]);
+    };
+    const int nfast = max(0, p.K / kBK - (C::NS - 1));
+    int kt = 0;
+    for (; kt < nfast; ++kt) iter(kt, std::true_type{});
+    for (; kt < nk; ++kt) iter(kt, std::false_type{});
+  };
+  const int live = row_end - row0;
+  if (C::FR >= 2 && live <= 32)
+    main_loop(std::integral_constant<int, 1>{});
+  else if (C::FR >= 4 && live <= 64)
+    main_loop(std::integral_constant<int, 2>{});
+  else
+    main_loop(std::integral_constant<int, C::FR>{});
+  wait_vm<0>();
+
+  // ---- epilogue: a lane holds row a*32 + lane%32 and, per group g, 4 consecutive columns; it stores them itself (8
+  // bytes: with few rows the outputs are a few percent of the weights' bytes) ----
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    const int lc = wave * 32 + 8 * g + 4 * (lane >> 5);  // column within a 64-column half of the tile
+    if constexpr (EPI == EPI_SWIGLU) {
+      const int col = n0 + lc;
+      if (col >= p.N) continue;
+#pragma unroll
+      for (int a = 0; a < C::FR; ++a) {
+        const int64_t row = row0 + a * 32 + (lane & 31);
+        if (row >= row_end) continue;
+        float gs[4], us[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          gs[t] = acc[a][0][4 * g + t];
+          us[t] = acc[a][1][4 * g + t];
+          if constexpr (C::BE == 1) {
+            gs[t] *= cs[0][g][t];
+            us[t] *= cs[1][g][t];
+          }
+        }
+        // act = R(R(silu(g)) * u) with g, u the rounded projections (R: to bf16, or fp16 with F16)
+        uint32_t o[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          const uint32_t gb = X::pack2(gs[2 * t], gs[2 * t + 1]), ub = X::pack2(us[2 * t], us[2 * t + 1]);
+          const uint32_t sl = X::pack2(silu_f(X::lo(gb)), silu_f(X::hi(gb)));
+          o[t] = X::pack2(X::lo(sl) * X::lo(ub), X::hi(sl) * X::hi(ub));
+        }
+        *reinterpret_cast<uint2*>(static_cast<uint16_t*>(p.C) + row * p.ldc + col) = make_uint2(o[0], o[1]);
+      }
+    } else {
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        const int col = n0 + C::BN / 2 * b + lc;
+        if (col >= p.N) continue;
+#pragma unroll
+        for (int a = 0; a < C::FR; ++a) {
+          const int64_t row = row0 + a * 32 + (lane & 31);
+          if (row >= row_end) continue;
+          float v[4];
+#pragma unroll
+          for (int t = 0; t < 4; ++t) {
+            v[t] = acc[a][b][4 * g + t];
+            if constexpr (C::BE == 1) v[t] *= cs[b][g][t];  // the column scale first, then the row scale
+            v[t] *= sc[a];
+          }
+          *reinterpret_cast<uint2*>(static_cast<uint16_t*>(p.C) + (int64_t)yr[a] * p.ldc + col) =
+              make_uint2(X::pack2(v[0], v[1]), X::pack2(v[2], v[3]));
+        }
+      }
+    }
+  }
+}
+
+}  // namespace hmoe
