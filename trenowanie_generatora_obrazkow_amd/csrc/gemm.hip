@@ -1071,16 +1071,16 @@ static inline int64_t cu_count() {
 // about 1.5x less per flop than two co-resident small ones, so large tiles win unless they leave too few tiles to
 // spread over the CUs or pad much more of the output.
 //
-// Row-grouped launches (bf16 weights): large tiles from 5/8 of a tile per CU on (160 tiles on 256 CUs): at 64-128
-// tiles small ones ran 15-55% faster, from 160 tiles on large ones ran 10-57% faster, also at K = 320 (the h = 320
-// down GEMM, 20-47%).  int8 weights: large tiles only with K of at least 16 slices (the h = 320 down GEMM ran 5-25%
-// faster on small int8 tiles) and, for the gate/up GEMM, from 2.5 tiles per CU (at 384-576 tiles the small int8
-// tiles ran up to 34% faster).  Either way, once the large tiles give two per CU, small ones where the large would
-// pad the output columns by more than 10% (a SwiGLU n-tile with at most 64 live columns of 128 counts as 64: its
-// main loop skips the dead half); with fewer tiles the rounds they save matter more (the h = 320 down dgrad ran 53%
-// faster on large tiles at 2048 tokens, 3% slower at 8192).
+// Row-grouped launches: large tiles from 5/8 of a tile per CU on (160 tiles on 256 CUs): at 64-128 tiles small ones ran
+// 15-55% faster, from 160 tiles on large ones ran 10-57% faster, also at K = 320 (the h = 320 down GEMM, 20-47%).  int8
+// weights follow the same line since their conversions run in the MFMAs' shadow (large against small tiles, us: 128 experts,
+// h 320, 192 rows each gate/up 93 / 121 and down 75 / 86, 512 rows 210 / 258 and 198 / 198; 64 experts, h 1408, 192 rows
+// 174 / 244 and 89 / 120).  Once the large tiles give two per CU, small ones where the large would pad the output columns
+// by more than 10% (a SwiGLU n-tile with at most 64 live columns of 128 counts as 64: its main loop skips the dead half);
+// with fewer tiles the rounds they save matter more (the h = 320 down dgrad ran 53% faster on large tiles at 2048 tokens,
+// 3% slower at 8192).
 template <int EPI>
-static bool pick_large_mgroup(int64_t tiles_large, int64_t ncols, int64_t K, bool int8) {
+static bool pick_large_mgroup(int64_t tiles_large, int64_t ncols) {
   const int f = env_force();
   if (f) return f == 1;
   const int64_t cus = cu_count();
@@ -1091,15 +1091,13 @@ static bool pick_large_mgroup(int64_t tiles_large, int64_t ncols, int64_t K, boo
     if (EPI == EPI_SWIGLU && ncols % bl && ncols % bl <= bl / 2) padl -= bl / 2;
     if (padl * 10 > pads * 11) return false;
   }
-  if (!int8) return tiles_large * 8 >= cus * 5;
-  if (K < 16 * kBK) return false;
-  return EPI == EPI_SWIGLU ? tiles_large * 2 >= cus * 5 : tiles_large * 8 >= cus * 5;
+  return tiles_large * 8 >= cus * 5;
 }
 
 template <int MODE, bool A_MN, bool B_MN, int EPI, bool A_BLK = false, bool F16 = false>
 static int launch_mgroup(const GemmParams& p, int64_t ncols, hipStream_t s) {
   const int64_t tl = mgroup_tiles<CfgL, EPI>(p.M, p.E, ncols);
-  if (pick_large_mgroup<EPI>(tl, ncols, p.K, false))
+  if (pick_large_mgroup<EPI>(tl, ncols))
     return launch<CfgL, MODE, A_MN, B_MN, EPI, A_BLK, F16>(p, tl, s);
   return launch<CfgS, MODE, A_MN, B_MN, EPI, A_BLK, F16>(p, mgroup_tiles<CfgS, EPI>(p.M, p.E, ncols), s);
 }
@@ -1124,19 +1122,20 @@ static int launch_few_tile(const GemmParams& p, int64_t ncols, hipStream_t s) {
   return HMOE_OK;
 }
 
-// The few-rows kernel (gemm_few.h) or the persistent one.  Measured on MI355X over 8 layers (d 256-2048, h 320-4096, 1-128
-// experts, bf16, fp16 and int8 weights), 2 to 256 routed rows per expert, gate/up and down, every tile against the
-// persistent kernel's choice in one process; us, persistent -> few:
-//   d 2048, h 320, 128 int8 experts: 4 rows per expert 59.5 -> 31.7 (gate/up) and 34.4 -> 24.3 (down), 32 rows 60 -> 37
-//   and 35.5 -> 28.5, 96 rows 69.9 -> 57.7 and 41.9 -> 42.5; d 2048, h 1408, 64 int8 experts: 2 rows 92.8 -> 59.7 and
-//   48 -> 32, 96 rows 129 -> 109 and 59.7 -> 50.7; d 1536, h 1024, 60 fp16 experts: 48 rows 79.1 -> 75.5 and 45 -> 36.8,
-//   96 rows 88.5 -> 83.4 and 50.2 -> 44.6; d 256, h 512, 8 experts: 128 rows 8.8 -> 7.3 and 10.1 -> 7.8.
-// Tiles: 64 rows x 256 columns up to 52 rows per expert (above, most experts need a second tile, which reads the weights
-// again), then 128 x 256, or 64 x 256 where those leave too few workgroups.  Where even a third of a workgroup per CU is
-// not reached, 32 x 128, while these give no more than 3/4 of a workgroup per CU (1.5 with K up to 512: the launch is
-// then a handful of latencies long).  Above 144 (int8) or 112 rows per expert the products bound the launch and the
-// persistent kernel's 256-row tiles win (128 rows: fp16 gate/up 92.8 against 99.8, int8 154.5 against 129.7; 192 rows:
-// int8 176 against 204).
+// The few-rows kernel (gemm_few.h) or the persistent one.  Measured on MI355X over 10 layers (d 256-2048, h 320-4096, 1-128
+// experts, bf16, fp16 and int8 weights), 2 to 768 routed rows per expert, gate/up and down, every tile against the
+// persistent kernel in one process, the weights of successive calls apart (read from HBM); us, persistent -> few:
+//   d 2048, h 320, 128 int8 experts: 8 rows per expert 61.8 -> 43.5 (gate/up) and 37.6 -> 27.6 (down), 48 rows 65.6 -> 55.4
+//   and 40 -> 34.4, 94 rows 78.8 -> 69.3 and 49.7 -> 49.8; d 2048, h 1408, 64 int8 experts: 2 rows 93 -> 67 and 50 -> 35,
+//   94 rows 121 -> 107 and 66 -> 57; d 1536, h 1024, 60 fp16 experts: 24 rows 75.9 -> 73 and 49 -> 44, 94 rows 87.8 -> 82.5
+//   and 57.2 -> 55.5; d 256, h 512, 8 experts: 94 rows 9.0 -> 6.9 and 10.0 -> 7.9.
+// Tiles: 64 rows x 256 columns up to 52 (16-bit weights: 40) rows per expert, above which experts often need a second tile,
+// which reads the weights again (48 rows, h 1408, int8 gate/up: 82 against 100 with 128-row tiles, whose copies of A cost
+// more beside half the weight bytes; 16-bit 76.0 / 76.2); then 128 x 256, or 64 x 256 where those leave too few workgroups.
+// 32 x 128 where they give no more than 3/4 of a workgroup per CU (1.5 with K up to 512: the launch is then a handful of
+// latencies long).  Above 112 (int8 gate/up: 132) rows per expert the products bound the launch and the persistent kernel's
+// 256-row tiles win (128 rows: fp16 gate/up 94 against 110, int8 down 64 / 68 and 75 / 84, int8 gate/up 89 / 77 and 148 /
+// 138; 160 rows: int8 gate/up 89 / 104 and 166 / 188).
 enum FewTile { FEW_NONE, FEW_32x128, FEW_64x256, FEW_128x256 };
 template <int EPI>
 static FewTile pick_few(int64_t M, int64_t E, int64_t ncols, int64_t K, bool int8) {
@@ -1148,8 +1147,8 @@ static FewTile pick_few(int64_t M, int64_t E, int64_t ncols, int64_t K, bool int
   };
   const int64_t ta = tiles(32, 128);
   if (ta * 4 <= cus * 3 || (ta * 2 <= cus * 3 && K <= 512)) return FEW_32x128;
-  if (M > E * (int8 ? 144 : 112)) return FEW_NONE;
-  if (M > E * 52 && tiles(128, 256) >= cus) return FEW_128x256;
+  if (M > E * (int8 && EPI == EPI_SWIGLU ? 132 : 112)) return FEW_NONE;
+  if (M > E * (int8 ? 52 : 40) && tiles(128, 256) >= cus) return FEW_128x256;
   return tiles(64, 256) * 8 >= cus * 3 ? FEW_64x256 : FEW_NONE;
 }
 
@@ -1186,14 +1185,7 @@ static int launch_mgroup_i8_t(const GemmParams& p, int64_t ncols, hipStream_t s)
   const int rc = launch_few<EPI, F16, 1>(p, ncols, s, &done);
   if (done) return rc;
   const int64_t tl = mgroup_tiles<CfgL8, EPI>(p.M, p.E, ncols);
-  bool large = pick_large_mgroup<EPI>(tl, ncols, p.K, true);
-  // gate/up with many experts (E >= 128): the tile bound counts a partial tile per expert, and below 3.25 large
-  // tiles per CU by it the small tiles ran faster (E = 128, h = 320, top-8, 4096 tokens, bound 3.0: gate/up 186 ->
-  // 166 us, the BailingMoeV2 block 407 -> 379 us).  At 5120 tokens (3.375) the gate/up alone still ran 5% faster
-  // on small tiles but the block, where it shares the CUs with the shared expert, 5% slower; at 3.75 the large
-  // tiles ran 5% faster alone.  With 16 or 64 experts the large tiles stay ahead over that range.
-  if (large && EPI == EPI_SWIGLU && !env_force() && p.E >= 128 && tl * 4 < cu_count() * 13) large = false;
-  if (large) return launch<CfgL8, MGROUP, false, true, EPI, false, F16>(p, tl, s);
+  if (pick_large_mgroup<EPI>(tl, ncols)) return launch<CfgL8, MGROUP, false, true, EPI, false, F16>(p, tl, s);
   return launch<CfgS8, MGROUP, false, true, EPI, false, F16>(p, mgroup_tiles<CfgS8, EPI>(p.M, p.E, ncols), s);
 }
 template <int EPI>
@@ -1527,7 +1519,7 @@ int hmoe_down_dgrad_swiglu_dw(const void* dy, const int32_t* a_idx, const uint16
     return HMOE_ERR_WORKSPACE;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const int64_t tl = mgroup_tiles<CfgL, EPI_SWIGLU_BWD>(M, E, h);
-  const bool large = pick_large_mgroup<EPI_SWIGLU_BWD>(tl, h, d, false);
+  const bool large = pick_large_mgroup<EPI_SWIGLU_BWD>(tl, h);
   p.dw_part = static_cast<float*>(workspace);
   p.dw_ld = (int)dw_partials(h, large);
   rc = large ? launch<CfgL, MGROUP, false, false, EPI_SWIGLU_BWD>(p, tl, s)

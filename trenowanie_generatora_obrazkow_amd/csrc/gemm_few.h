@@ -15,8 +15,9 @@
 // The products and their order in k are those of the persistent kernel (the same 32x32x16 MFMAs in k order from zero), and
 // so are the roundings of the epilogues: the results are bit-identical.
 //
-// Measured (GB/s of weights read once): 24 tokens, top-6 of 64 int8 experts, d 2048, h 1408: gate/up 90 -> 59 us (5650),
-// down 47.5 -> 30.8 (5400); 64 tokens, top-8 of 128, h 320: 58 -> 31 (5400) and 34 -> 23.6 (3560).
+// Measured inside whole calls whose weights come from HBM (GB/s of weights): 24 tokens, top-6 of 64 int8 experts, d 2048,
+// h 1408: gate/up 126 -> 66.7 us (5000), down 63 -> 36.4 (4600); 64 tokens, top-8 of 128, h 320: 68.8 -> 43.2 (3900) and
+// 37.2 -> 27.3 (3070).
 #pragma once
 #include "gemm_common.h"
 
