@@ -283,6 +283,13 @@ int hmoe_down_dgrad_swiglu_dw(const void* dy, const int32_t* a_idx, const uint16
 int hmoe_gate_up_dgrad(const void* dgu, const void* wgu, int64_t E, int64_t d, int64_t h, const void* counts,
                        int counts_dtype, int64_t M, void* dxs, int dxs_dtype, hmoe_stream_t stream);
 
+/* The same with the reduction over 2h split into `parts` (fp32, each part's sum in its own (M, d) of dxs (parts, M, d)), for
+ * row counts whose output has too few tiles to fill the chip; hmoe_unpermute_bwd_split adds the parts as it reads them.
+ * hmoe_gate_up_dgrad_parts says how many parts these sizes are best split into (1: do not split). */
+int hmoe_gate_up_dgrad_parts(int64_t M, int64_t E, int64_t d, int64_t h);
+int hmoe_gate_up_dgrad_split(const void* dgu, const void* wgu, int64_t E, int64_t d, int64_t h, const void* counts,
+                             int counts_dtype, int64_t M, float* dxs, int parts, hmoe_stream_t stream);
+
 /* Weight gradients of :79 and :81: dw[e] = a[rows of e]^T @ b[rows of e] (fp32 accumulation over the expert's
  * ragged row range, no split, deterministic); a (M, P) row stride lda, b (M, N) row stride ldb, both bf16 in
  * sorted order; dw (E, P, N) fp32 or bf16 (dw_dtype).  Experts with no rows get zeros (M = 0: all of dw, and a,
@@ -307,6 +314,10 @@ int hmoe_router_bwd(const float* logits, const int32_t* topk_ids, const float* d
  * only); dxs (M, d) bf16 or fp32 (dxs_dtype); slots with a negative inv_pos add nothing. */
 int hmoe_unpermute_bwd(const void* dxs, int dxs_dtype, const int32_t* inv_pos, const float* dlogits, const void* wr,
                        int64_t T, int k, int64_t d, int E, void* dx, hmoe_stream_t stream);
+
+/* The same from the parts of hmoe_gate_up_dgrad_split: dxs (parts, T k, d) fp32, added in order. */
+int hmoe_unpermute_bwd_split(const float* dxs, int parts, const int32_t* inv_pos, const float* dlogits, const void* wr,
+                             int64_t T, int k, int64_t d, int E, void* dx, hmoe_stream_t stream);
 
 #ifdef __cplusplus
 }

@@ -59,11 +59,14 @@ SIGNATURES = {
     "hmoe_down_dgrad_swiglu_dw": (_I32, [_P, _P, _P, _P, _I64, _I64, _I64, _P, _I32, _I64, _P, _P, _P, _P, _P, _SZ,
                                          _P]),
     "hmoe_gate_up_dgrad": (_I32, [_P, _P, _I64, _I64, _I64, _P, _I32, _I64, _P, _I32, _P]),
+    "hmoe_gate_up_dgrad_parts": (_I32, [_I64, _I64, _I64, _I64]),
+    "hmoe_gate_up_dgrad_split": (_I32, [_P, _P, _I64, _I64, _I64, _P, _I32, _I64, _P, _I32, _P]),
     "hmoe_grouped_wgrad": (_I32, [_P, _I64, _P, _I64, _I64, _I64, _I64, _P, _I32, _I64, _P, _I32, _P]),
     "hmoe_router_bwd_workspace_size": (_SZ, [_I64, _I32, _I64]),
     "hmoe_router_bwd": (_I32, [_P, _P, _P, _I64, _I32, _I32, _I32, _F32, _P, _I64, _I64, _P, _P, _I32, _P, _SZ,
                                _P]),
     "hmoe_unpermute_bwd": (_I32, [_P, _I32, _P, _P, _P, _I64, _I32, _I64, _I32, _P, _P]),
+    "hmoe_unpermute_bwd_split": (_I32, [_P, _I32, _P, _P, _P, _I64, _I32, _I64, _I32, _P, _P]),
 }
 
 _lib = None

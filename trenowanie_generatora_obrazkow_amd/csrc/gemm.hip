@@ -122,7 +122,10 @@ __global__ __launch_bounds__(C::NT, 1) void grouped_gemm_kernel(GemmParams p) {
     nb_n = (p.N + C::BN - 1) / C::BN;
   const int nb_i = MODE == KGROUP ? (p.P + C::BM - 1) / C::BM : 1;
   const int total_m = MODE == MGROUP ? s_tstart[E] : E * nb_i;
-  const int total = total_m * nb_n;
+  // split reduction (EPI_STORE_F32): every tile once per part, all tiles of a part in a row
+  const int parts = EPI == EPI_STORE_F32 ? p.parts : 1;
+  const int part_tiles = total_m * nb_n;
+  const int total = part_tiles * parts;
 
   typename TileSel<A_MN, C::BM, C::NWAVES>::type ta;
   typename TileSel<B_MN, C::BN, C::NWAVES, C::BE, C::FN, F16>::type tb;
@@ -156,6 +159,11 @@ __global__ __launch_bounds__(C::NT, 1) void grouped_gemm_kernel(GemmParams p) {
     }
     // ---- tile decode ----
     int mt, nb;
+    [[maybe_unused]] int part = 0;
+    if constexpr (EPI == EPI_STORE_F32) {
+      part = tile / part_tiles;
+      tile -= part * part_tiles;
+    }
     {
       const int per_group = C::GM * nb_n;  // bands of GM m-tiles x all n-tiles
       // Band residency.  With the XCD-aware slots, XCD x runs tiles [r G + x G/8, r G + (x+1) G/8) in round r: one
@@ -165,7 +173,7 @@ __global__ __launch_bounds__(C::NT, 1) void grouped_gemm_kernel(GemmParams p) {
       // A rows in its L2.  Only the order in which workgroups take tiles changes, not what a tile computes.  (Not for
       // the weight gradients: their bands' A columns, 4 MB at the C5 shape, do not stay in a 4 MB L2, and the order
       // measured slower there.)
-      if (MODE == MGROUP && (G & 7) == 0) {
+      if (MODE == MGROUP && (G & 7) == 0 && parts == 1) {
         const int XB = G >> 3;
         if (per_group % XB == 0) {
           const int BPB = per_group / XB, SG = 8 * BPB;  // blocks per band, per super-group
@@ -184,7 +192,8 @@ __global__ __launch_bounds__(C::NT, 1) void grouped_gemm_kernel(GemmParams p) {
     int64_t row0 = 0, row_end = 0;  // MGROUP: sorted rows [row0, row_end) of this m-tile's expert
     int i0 = 0;                     // KGROUP: first output row
     int64_t kstart = 0;
-    int kvalid = p.K;
+    const int k0 = EPI == EPI_STORE_F32 ? part * p.kper : 0;  // the part's first k, and its length
+    int kvalid = EPI == EPI_STORE_F32 ? min(p.K - k0, p.kper) : p.K;
     if (MODE == MGROUP) {
       int lo = 0, hi = E;  // largest e with s_tstart[e] <= mt (empty experts share the start of the next)
       while (hi - lo > 1) {
@@ -217,7 +226,7 @@ __global__ __launch_bounds__(C::NT, 1) void grouped_gemm_kernel(GemmParams p) {
     // ---- copy sources for this tile (buffer bases and per-lane byte offsets) ----
     if constexpr (MODE == MGROUP) {
       static_assert(!A_MN, "MGROUP A is K-contiguous");
-      ta.K = p.K;
+      ta.K = kvalid;
       if constexpr (A_BLK) {
         // row-group tiles: instruction I's 16 rows (tile rows 16 I ..) are one 1 KB run of their group's slice
         ta.kmul = kTileSliceBytes / kBK;
@@ -236,7 +245,7 @@ __global__ __launch_bounds__(C::NT, 1) void grouped_gemm_kernel(GemmParams p) {
         }
       } else {
         // gathered rows are addressed from A itself; contiguous rows from the tile's first row
-        ta.rsrc = make_rsrc(p.a_idx ? p.A : p.A + row0 * p.lda);
+        ta.rsrc = make_rsrc((p.a_idx ? p.A : p.A + row0 * p.lda) + k0);
 #pragma unroll
         for (int i = 0; i < ta.PER_WAVE; ++i) {
           const int rr = ta.row_of(wave, lane, i);
@@ -251,7 +260,8 @@ __global__ __launch_bounds__(C::NT, 1) void grouped_gemm_kernel(GemmParams p) {
           ta.chunk[i] = c;
         }
       }
-      tb.rsrc = make_rsrc(static_cast<const char*>(p.B) + (int64_t)e * p.strideBe * C::BE);
+      static_assert(EPI != EPI_STORE_F32 || !B_MN, "a split reduction advances B along a row");
+      tb.rsrc = make_rsrc(static_cast<const char*>(p.B) + ((int64_t)e * p.strideBe + k0) * C::BE);
       auto gcol = [&](int nn, int& col) -> bool {  // tile column -> weight column
         if (EPI == EPI_SWIGLU) {
           const int half = nn / (C::BN / 2);  // tile columns [0, BN/2) gate, [BN/2, BN) the matching up
@@ -265,7 +275,7 @@ __global__ __launch_bounds__(C::NT, 1) void grouped_gemm_kernel(GemmParams p) {
       };
       if constexpr (B_MN) {
         tb.kstep = (uint32_t)(p.ldb * C::BE);
-        tb.Kvalid = p.K;
+        tb.Kvalid = kvalid;
 #pragma unroll
         for (int i = 0; i < tb.PER_WAVE; ++i) {
           int k, nn, col;
@@ -275,7 +285,7 @@ __global__ __launch_bounds__(C::NT, 1) void grouped_gemm_kernel(GemmParams p) {
         }
       } else {
         static_assert(C::BE == 2, "int8 weights are read N-contiguous only");
-        tb.K = p.K;
+        tb.K = kvalid;
 #pragma unroll
         for (int i = 0; i < tb.PER_WAVE; ++i) {
           const int nn = tb.row_of(wave, lane, i);
@@ -839,7 +849,8 @@ __global__ __launch_bounds__(C::NT, 1) void grouped_gemm_kernel(GemmParams p) {
           return (p.y_idx ? (int64_t)s_rowy[par][rt + y_sh] : row) * p.ldc * ES;
         });
         constexpr std::bool_constant<C::BE == 1> paired{};  // int8 weights: paired reads (bf16: one by one)
-        drain_rows(std::integral_constant<int, NSP>{}, 0, RB, ES, reinterpret_cast<char*>(p.C), rows, p.N, paired);
+        drain_rows(std::integral_constant<int, NSP>{}, 0, RB, ES,
+                   reinterpret_cast<char*>(p.C) + (EPI == EPI_STORE_F32 ? part * p.M * p.ldc * ES : 0), rows, p.N, paired);
         if constexpr (C::BE == 2) {
           if (aux)
             drain_rows(std::integral_constant<int, (C::FN * 32 * 2 + 127) / 128>{}, NSP, C::FN * 32 * 2, 2,
@@ -1235,6 +1246,7 @@ static GemmParams base_params(const void* counts, int counts_dtype, int64_t E, i
   p.counts64 = counts_dtype == HMOE_DT_I64;
   p.E = (int)E;
   p.M = M;
+  p.parts = 1;
   return p;
 }
 
@@ -1531,8 +1543,22 @@ int hmoe_down_dgrad_swiglu_dw(const void* dy, const int32_t* a_idx, const uint16
   return HMOE_OK;
 }
 
-int hmoe_gate_up_dgrad(const void* dgu, const void* wgu, int64_t E, int64_t d, int64_t h, const void* counts,
-                       int counts_dtype, int64_t M, void* dxs, int dxs_dtype, hmoe_stream_t stream) {
+// Parts of the gate/up dgrad's reduction (K = 2h).  Its output is narrow (d), so a few thousand rows give far fewer 256x256
+// tiles than there are CUs; 128x128 tiles fill the chip, but read both operands in 64-byte pieces twice as often and ran
+// 1.5x slower per flop.  Where the tile rule would leave the large ones, the reduction is split into up to four parts of
+// them instead, as many as fit one round (half a tile more per expert than whole ones, 2% to spare), each part at least 512 deep;
+// whoever reads the rows adds the parts.
+int hmoe_gate_up_dgrad_parts(int64_t M, int64_t E, int64_t d, int64_t h) {
+  if (M <= 0 || E <= 0 || d <= 0 || h <= 0) return 1;
+  if (env_force() || pick_large_mgroup<EPI_STORE_F32>(mgroup_tiles<CfgL, EPI_STORE_F32>(M, E, d), d)) return 1;
+  const int64_t nt = (d + CfgL::BN - 1) / CfgL::BN, half_tiles = (2 * (M / CfgL::BM) + std::min(E, M)) * nt;
+  const int64_t fit = cu_count() * 49 / (25 * half_tiles), deep = 2 * h / 512;
+  return (int)std::max<int64_t>(1, std::min({fit, deep, (int64_t)4}));
+}
+
+// parts > 1: large tiles, dxs (parts, M, d) fp32
+static int gate_up_dgrad(const void* dgu, const void* wgu, int64_t E, int64_t d, int64_t h, const void* counts,
+                         int counts_dtype, int64_t M, void* dxs, int dxs_dtype, int parts, hmoe_stream_t stream) {
   int rc = check_common(counts, counts_dtype, E, M);
   if (rc) return rc;
   if (M == 0) return HMOE_OK;
@@ -1541,6 +1567,8 @@ int hmoe_gate_up_dgrad(const void* dgu, const void* wgu, int64_t E, int64_t d, i
   if (d % 8 || h % 8) return HMOE_ERR_SHAPE;
   if (!al16(dgu) || !al16(wgu) || !al16(dxs)) return HMOE_ERR_ARG;
   if (!off32(d * 2 * h * 2)) return HMOE_ERR_SHAPE;
+  const int64_t slices = (2 * h + kBK - 1) / kBK;
+  if (parts < 1 || parts > slices || M * parts > INT32_MAX) return HMOE_ERR_ARG;
   GemmParams p = base_params(counts, counts_dtype, E, M);
   p.A = static_cast<const uint16_t*>(dgu);
   p.lda = 2 * h;
@@ -1551,9 +1579,23 @@ int hmoe_gate_up_dgrad(const void* dgu, const void* wgu, int64_t E, int64_t d, i
   p.N = (int)d;
   p.C = dxs;
   p.ldc = d;
-  if (dxs_dtype == HMOE_DT_F32)
-    return launch_mgroup<MGROUP, false, false, EPI_STORE_F32>(p, d, reinterpret_cast<hipStream_t>(stream));
-  return launch_mgroup<MGROUP, false, false, EPI_STORE>(p, d, reinterpret_cast<hipStream_t>(stream));
+  p.kper = (int)((slices + parts - 1) / parts * kBK);
+  p.parts = (int)((slices * kBK + p.kper - 1) / p.kper);
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  if (p.parts != parts) return HMOE_ERR_ARG;  // (a part without a slice: dxs would not be written whole)
+  if (dxs_dtype != HMOE_DT_F32) return launch_mgroup<MGROUP, false, false, EPI_STORE>(p, d, s);
+  if (parts == 1) return launch_mgroup<MGROUP, false, false, EPI_STORE_F32>(p, d, s);
+  return launch<CfgL, MGROUP, false, false, EPI_STORE_F32>(p, mgroup_tiles<CfgL, EPI_STORE_F32>(M, E, d) * parts, s);
+}
+
+int hmoe_gate_up_dgrad(const void* dgu, const void* wgu, int64_t E, int64_t d, int64_t h, const void* counts,
+                       int counts_dtype, int64_t M, void* dxs, int dxs_dtype, hmoe_stream_t stream) {
+  return gate_up_dgrad(dgu, wgu, E, d, h, counts, counts_dtype, M, dxs, dxs_dtype, 1, stream);
+}
+
+int hmoe_gate_up_dgrad_split(const void* dgu, const void* wgu, int64_t E, int64_t d, int64_t h, const void* counts,
+                             int counts_dtype, int64_t M, float* dxs, int parts, hmoe_stream_t stream) {
+  return gate_up_dgrad(dgu, wgu, E, d, h, counts, counts_dtype, M, dxs, HMOE_DT_F32, parts, stream);
 }
 
 int hmoe_grouped_wgrad(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t E, int64_t P, int64_t N,

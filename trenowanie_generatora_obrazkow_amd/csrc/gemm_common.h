@@ -396,6 +396,8 @@ struct GemmParams {
   const void* w_scale;      // int8 weights: per-(expert, column) scale (E, ldws), bf16 or fp32
   int w_scale_f32;
   int64_t ldws;             // scale row length (columns of the weight)
+  int parts;                // EPI_STORE_F32: the reduction split into this many parts of kper, each its own C (M, N)
+  int kper;                 //   (a multiple of the slice)
 };
 
 }  // namespace hmoe

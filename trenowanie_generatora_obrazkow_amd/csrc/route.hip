@@ -1716,13 +1716,16 @@ __global__ __launch_bounds__(1024) void router_dwr_reduce_kernel(const float* __
 
 // dx[t] = bf16(sum_j dxs[inv_pos[t*k+j]] + sum_e dlogits[t,e] * wr[e]).  A workgroup walks tokens; each thread owns
 // 8 columns of a column slab (blockIdx.y), so the token's row indices and router gradients are wave-uniform scalar
-// loads.  EMAX > 0: the thread's wr columns for E <= EMAX experts stay in registers for all its tokens.
-template <bool F32, int EMAX>
+// loads.  EMAX > 0: the thread's wr columns for E <= EMAX experts stay in registers for all its tokens.  SPLIT: dxs comes in
+// `parts` fp32 arrays of T k rows each (a split reduction), added in order.
+template <bool F32, int EMAX, bool SPLIT = false>
 __global__ __launch_bounds__(256) void unpermute_bwd_kernel(const void* __restrict__ dxs,
                                                             const int32_t* __restrict__ inv_pos,
                                                             const float* __restrict__ dlogits,
                                                             const uint16_t* __restrict__ wr, int64_t T, int k,
-                                                            int64_t d, int E, uint16_t* __restrict__ dx) {
+                                                            int64_t d, int E, uint16_t* __restrict__ dx,
+                                                            int parts) {
+  static_assert(F32 || !SPLIT, "parts are fp32");
   const int64_t col = ((int64_t)blockIdx.y * blockDim.x + threadIdx.x) * 8;
   const bool active = col < d;
   [[maybe_unused]] uint4 wreg[EMAX > 0 ? EMAX : 1];
@@ -1758,6 +1761,21 @@ __global__ __launch_bounds__(256) void unpermute_bwd_kernel(const void* __restri
           s[u][5] += v1.y;
           s[u][6] += v1.z;
           s[u][7] += v1.w;
+          if constexpr (SPLIT) {
+            for (int q = 1; q < parts; ++q) {
+              const float4* more = reinterpret_cast<const float4*>(static_cast<const float*>(dxs) +
+                                                                   ((int64_t)q * T * k + r) * d + col);
+              const float4 w0 = more[0], w1 = more[1];
+              s[u][0] += w0.x;
+              s[u][1] += w0.y;
+              s[u][2] += w0.z;
+              s[u][3] += w0.w;
+              s[u][4] += w1.x;
+              s[u][5] += w1.y;
+              s[u][6] += w1.z;
+              s[u][7] += w1.w;
+            }
+          }
         } else {
           const uint4 v = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(dxs) + r * d + col);
           const uint32_t w[4] = {v.x, v.y, v.z, v.w};
@@ -2284,9 +2302,9 @@ int hmoe_router_bwd(const float* logits, const int32_t* topk_ids, const float* d
   return HMOE_OK;
 }
 
-int hmoe_unpermute_bwd(const void* dxs, int dxs_dtype, const int32_t* inv_pos, const float* dlogits, const void* wr,
-                       int64_t T, int k, int64_t d, int E, void* dx, hmoe_stream_t stream) {
-  if (T < 0 || k <= 0 || d <= 0) return HMOE_ERR_ARG;
+static int unpermute_bwd(const void* dxs, int dxs_dtype, int parts, const int32_t* inv_pos, const float* dlogits,
+                         const void* wr, int64_t T, int k, int64_t d, int E, void* dx, hmoe_stream_t stream) {
+  if (T < 0 || k <= 0 || d <= 0 || parts < 1) return HMOE_ERR_ARG;
   if (T == 0) return HMOE_OK;
   if (dxs_dtype != HMOE_DT_BF16 && dxs_dtype != HMOE_DT_F32) return HMOE_ERR_DTYPE;
   if (!dxs || !inv_pos || !dx || d % 8 || !al16(dxs) || !al16(dx)) return HMOE_ERR_ARG;
@@ -2300,10 +2318,15 @@ int hmoe_unpermute_bwd(const void* dxs, int dxs_dtype, const int32_t* inv_pos, c
   const uint16_t* wp = static_cast<const uint16_t*>(wr);
   uint16_t* dxp = static_cast<uint16_t*>(dx);
   const bool regs = dlogits == nullptr || E <= 16;
-#define HMOE_UNPERM(F, EM)                                                                                         \
-  hipLaunchKernelGGL((unpermute_bwd_kernel<F, EM>), dim3(tgrid, slabs), dim3(threads), 0, s, dxs, inv_pos, dlogits, \
-                     wp, T, k, d, E, dxp)
-  if (dxs_dtype == HMOE_DT_F32) {
+#define HMOE_UNPERM(...)                                                                                     \
+  hipLaunchKernelGGL((unpermute_bwd_kernel<__VA_ARGS__>), dim3(tgrid, slabs), dim3(threads), 0, s, dxs, inv_pos, \
+                     dlogits, wp, T, k, d, E, dxp, parts)
+  if (parts > 1) {
+    if (regs)
+      HMOE_UNPERM(true, 16, true);
+    else
+      HMOE_UNPERM(true, 0, true);
+  } else if (dxs_dtype == HMOE_DT_F32) {
     if (regs)
       HMOE_UNPERM(true, 16);
     else
@@ -2317,6 +2340,16 @@ int hmoe_unpermute_bwd(const void* dxs, int dxs_dtype, const int32_t* inv_pos, c
 #undef HMOE_UNPERM
   HMOE_CHECK_LAUNCH();
   return HMOE_OK;
+}
+
+int hmoe_unpermute_bwd(const void* dxs, int dxs_dtype, const int32_t* inv_pos, const float* dlogits, const void* wr,
+                       int64_t T, int k, int64_t d, int E, void* dx, hmoe_stream_t stream) {
+  return unpermute_bwd(dxs, dxs_dtype, 1, inv_pos, dlogits, wr, T, k, d, E, dx, stream);
+}
+
+int hmoe_unpermute_bwd_split(const float* dxs, int parts, const int32_t* inv_pos, const float* dlogits, const void* wr,
+                             int64_t T, int k, int64_t d, int E, void* dx, hmoe_stream_t stream) {
+  return unpermute_bwd(dxs, HMOE_DT_F32, parts, inv_pos, dlogits, wr, T, k, d, E, dx, stream);
 }
 
 }  // extern "C"

@@ -112,7 +112,8 @@ class _MoEFunction(torch.autograd.Function):
             dtw = dtw + dtw_out.to(torch.float32)
         if ctx.needs_input_grad[2]:
             dwgu = _to_param(ops.grouped_wgrad(xs, dgu, counts, E, dtype=_grad_dtype(wgu_dt)), wgu_dt)
-        dxs = ops.gate_up_dgrad(dgu, wgu, counts, M)
+        # (for a few thousand rows its reduction is split, and the un-permute adds the parts)
+        dxs = ops.gate_up_dgrad(dgu, wgu, counts, M, parts=ops.dgrad_parts(M, wgu))
         dl, dwr = ops.router_bwd(logits, ids, dtw, x, renorm=ctx.renorm, dwr_dtype=_grad_dtype(wr_dt),
                                  want_dwr=ctx.needs_input_grad[1])
         dwr = _to_param(dwr, wr_dt)

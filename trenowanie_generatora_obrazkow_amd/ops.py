@@ -577,15 +577,28 @@ def down_dgrad_swiglu_dw(dy, wd, counts, M, gu, order, k, a_idx=None, w_sorted=N
     return dgu, dtw
 
 
-def gate_up_dgrad(dgu, wgu, counts, M, dtype=torch.float32):
+def dgrad_parts(M, wgu):
+    """Parts the gate/up dgrad's reduction is best split into for M rows (1: not split)."""
+    E, d, h2 = wgu.shape
+    return L.lib().hmoe_gate_up_dgrad_parts(M, E, d, h2 // 2)
+
+
+def gate_up_dgrad(dgu, wgu, counts, M, dtype=torch.float32, parts=1):
+    """dxs (M, d) = dgu @ wgu[e]^T; parts > 1: (parts, M, d) fp32, the reduction split (unpermute_bwd adds the parts)."""
     _need(wgu, "wgu", (None, None, None), _BF16)
     E, d, h2 = wgu.shape
     counts = _counts(counts, E)
     _need(dgu, "dgu", (M, h2), _BF16)
-    dxs = torch.empty(M, d, device=dgu.device, dtype=dtype)
+    if parts > 1 and dtype != torch.float32:
+        raise TypeError(f"a split dgrad is fp32 (got {dtype})")
+    dxs = torch.empty((M, d) if parts == 1 else (parts, M, d), device=dgu.device, dtype=dtype)
     with _Probe("gate_up_dgrad"):
-        L.call("hmoe_gate_up_dgrad", L.ptr(dgu), L.ptr(wgu), E, d, h2 // 2, L.ptr(counts), L.dt(counts), M, L.ptr(dxs),
-               L.dt(dxs), _dev_stream(dgu))
+        if parts == 1:
+            L.call("hmoe_gate_up_dgrad", L.ptr(dgu), L.ptr(wgu), E, d, h2 // 2, L.ptr(counts), L.dt(counts), M,
+                   L.ptr(dxs), L.dt(dxs), _dev_stream(dgu))
+        else:
+            L.call("hmoe_gate_up_dgrad_split", L.ptr(dgu), L.ptr(wgu), E, d, h2 // 2, L.ptr(counts), L.dt(counts), M,
+                   L.ptr(dxs), parts, _dev_stream(dgu))
     return dxs
 
 
@@ -622,9 +635,14 @@ def router_bwd(logits, ids, dtw, x, renorm=True, scaling=1.0, dwr_dtype=torch.fl
 
 
 def unpermute_bwd(dxs, inv_pos, T, k, dlogits=None, wr=None):
-    d = dxs.shape[1]
+    """dx (T, d) bf16 from the sorted rows dxs (T*k, d), or the parts (parts, T*k, d) fp32 of a split gate_up_dgrad."""
+    parts = dxs.shape[0] if dxs.dim() == 3 else 1
+    d = dxs.shape[-1]
     E = wr.shape[0] if wr is not None else 0
-    _need(dxs, "dxs", (T * k, d), (torch.float32, torch.bfloat16))
+    if dxs.dim() == 3:
+        _need(dxs, "dxs", (None, T * k, d), (torch.float32,))
+    else:
+        _need(dxs, "dxs", (T * k, d), (torch.float32, torch.bfloat16))
     _need(inv_pos, "inv_pos", (T * k,), _I32)
     if (dlogits is None) != (wr is None):
         raise ValueError("dlogits and wr come together")
@@ -633,6 +651,10 @@ def unpermute_bwd(dxs, inv_pos, T, k, dlogits=None, wr=None):
         _need(dlogits, "dlogits", (T, E), (torch.float32,))
     dx = torch.empty(T, d, device=dxs.device, dtype=torch.bfloat16)
     with _Probe("unpermute_bwd"):
-        L.call("hmoe_unpermute_bwd", L.ptr(dxs), L.dt(dxs), L.ptr(inv_pos), L.ptr(dlogits), L.ptr(wr), T, k, d, E,
-               L.ptr(dx), _dev_stream(dxs))
+        if dxs.dim() == 3:
+            L.call("hmoe_unpermute_bwd_split", L.ptr(dxs), parts, L.ptr(inv_pos), L.ptr(dlogits), L.ptr(wr), T, k, d, E,
+                   L.ptr(dx), _dev_stream(dxs))
+        else:
+            L.call("hmoe_unpermute_bwd", L.ptr(dxs), L.dt(dxs), L.ptr(inv_pos), L.ptr(dlogits), L.ptr(wr), T, k, d, E,
+                   L.ptr(dx), _dev_stream(dxs))
     return dx
