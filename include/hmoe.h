@@ -247,6 +247,23 @@ int hmoe_moe_experts(const void* x, int64_t ldx, const void* topk_ids, int ids_d
                      void* y, int32_t* inv_pos, int32_t* n_invalid, void* workspace, size_t workspace_bytes,
                      int dtype, hmoe_stream_t stream);
 
+/* The whole BailingMoeV2 block in one call (inference, bf16): replaces aurora/hf_pipeline.py:348-370.  It runs
+ * hmoe_route_sigmoid_group, hmoe_moe_experts (bf16 or int8 experts) and hmoe_combine_add with the shared expert's output
+ * as the addend; the shared expert is hmoe_gate_up_swiglu and hmoe_down_scatter over one group of *sh_count = T rows,
+ * sh_wgu (d, 2 sh_h) = [gate | up], sh_wd (sh_h, d) bf16.  gate_w (E, d) bf16, expert_bias (E,) fp32 or NULL; out (T, d)
+ * bf16, the bits the entry points give one by one.  side: a second stream for the shared expert, or NULL to run it on
+ * `stream`; fork_event / join_event (without timing) order it: it starts when `stream` has reached this call, and
+ * `stream` waits for it before the combine, so nothing of this call is left running on `side` once `stream` has passed it.
+ * Calls that share the events may come from several threads.  workspace: hmoe_moe_block_workspace_size bytes, 256-byte
+ * aligned.  Limits as the entry points it runs. */
+size_t hmoe_moe_block_workspace_size(int64_t T, int64_t d, int E, int k, int64_t h, int64_t sh_h, int w_dtype);
+int hmoe_moe_block(const void* x, int64_t ldx, const void* gate_w, const float* expert_bias, int n_group,
+                   int topk_group, float scaling, const void* wgu, const void* wgu_s, int wgu_s_dtype, const void* wd,
+                   const void* wd_s, int wd_s_dtype, int w_dtype, const void* sh_wgu, const void* sh_wd,
+                   const int32_t* sh_count, int64_t sh_h, int64_t T, int64_t d, int E, int k, int64_t h, void* out,
+                   void* workspace, size_t workspace_bytes, hmoe_stream_t stream, hmoe_stream_t side, void* fork_event,
+                   void* join_event);
+
 /* ---------------------------------------------------------------------------------------------------------------
  * Backward.  The reference has no backward for this path (aurora/hf_compat.py:62 is @torch.no_grad); each entry
  * point below differentiates the forward line it names.

@@ -52,6 +52,9 @@ SIGNATURES = {
                                 _I32, _I64, _P, _P, _P, _P, _SZ, _I32, _P]),
     "hmoe_moe_forward": (_I32, [_P, _I64, _P, _P, _P, _P, _I64, _I64, _I32, _I32, _I64, _I32, _F32, _P, _P, _P, _P,
                                 _P, _SZ, _P]),
+    "hmoe_moe_block_workspace_size": (_SZ, [_I64, _I64, _I32, _I32, _I64, _I64, _I32]),
+    "hmoe_moe_block": (_I32, [_P, _I64, _P, _P, _I32, _I32, _F32, _P, _P, _I32, _P, _P, _I32, _I32, _P, _P, _P, _I64,
+                              _I64, _I64, _I32, _I32, _I64, _P, _P, _SZ, _P, _P, _P, _P]),
     "hmoe_combine_add": (_I32, [_P, _P, _I64, _I32, _I64, _P, _P, _I32, _P]),
     "hmoe_combine_bwd": (_I32, [_P, _P, _P, _P, _P, _I64, _I32, _I64, _P, _P, _P]),
     "hmoe_down_dgrad_swiglu": (_I32, [_P, _P, _P, _P, _I64, _I64, _I64, _P, _I32, _I64, _P, _P, _P]),

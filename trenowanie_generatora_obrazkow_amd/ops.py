@@ -33,7 +33,10 @@ def side_events(device: torch.device):
     and waited on in stream order, so one pair serves every fork (wait_stream would make a new event each time)."""
     key = device.index if device.index is not None else torch.cuda.current_device()
     if key not in _SIDE_EVENTS:
-        _SIDE_EVENTS[key] = (torch.cuda.Event(), torch.cuda.Event())
+        pair = (torch.cuda.Event(), torch.cuda.Event())
+        for ev in pair:  # an event's handle exists from its first record on
+            ev.record(torch.cuda.current_stream(key))
+        _SIDE_EVENTS[key] = pair
     return _SIDE_EVENTS[key]
 
 
@@ -224,6 +227,45 @@ def moe_experts(x, ids, tw, wgu, wd, wgu_s=None, wd_s=None):
            L.dt(wd_s) if wd_s is not None else 0, w_dt, T, d, E, k, h, L.ptr(y), L.ptr(inv), L.ptr(n_invalid),
            L.ptr(ws), ws_bytes, dt, _dev_stream(x))
     return y, inv, n_invalid
+
+
+def moe_block(x, gate_w, gate_b, k, n_group, topk_group, scaling, wgu, wgu_s, wd, wd_s, sh_wgu, sh_wd, sh_count,
+              overlap=True):
+    """The BailingMoeV2 block in one C call (hmoe_moe_block): route_sigmoid_group, moe_experts, the shared expert's
+    gate_up_swiglu and down_scatter (overlap: on the side stream), and the combine with its output, with the same
+    bits.  x (T, d) bf16 contiguous, T > 0; gate_w (E, d) bf16, gate_b (E,) fp32; wgu / wd bf16 or int8 with scales; sh_wgu
+    (1, d, 2h'), sh_wd (1, h', d) bf16; sh_count (1,) int32 = T -> out (T, d) bf16."""
+    T, d = x.shape
+    E = gate_w.shape[0]
+    _router_args(x, gate_w)
+    _need(gate_w, "router weight", (E, d))
+    _need(gate_b, "expert bias", (E,), (torch.float32,))
+    if wgu.dim() != 3 or wd.dim() != 3 or wgu.dtype not in (torch.bfloat16, torch.int8) or wd.dtype != wgu.dtype:
+        raise TypeError(f"wgu (E, d, 2h) and wd (E, h, d) of x's type or int8 expected (got {wgu.dtype}, {wd.dtype})")
+    h, sh = wd.shape[1], sh_wd.shape[1]
+    L.require_gpu(x, "x")
+    _need(wgu, "wgu", (E, d, 2 * h))
+    _need(wd, "wd", (E, h, d))
+    wgu_s = _w_scale(wgu, wgu_s, 2 * h)
+    wd_s = _w_scale(wd, wd_s, d)
+    _need(sh_wgu, "shared gate/up", (1, d, 2 * sh), _BF16)
+    _need(sh_wd, "shared down", (1, sh, d), _BF16)
+    w_dt = L.dt(wgu)
+    ws_bytes = L.lib().hmoe_moe_block_workspace_size(T, d, E, k, h, sh, w_dt)
+    if ws_bytes == 0:
+        raise ValueError(f"moe_block: unsupported sizes T={T} d={d} E={E} k={k} h={h} shared={sh}")
+    dev = x.device
+    ws = torch.empty(ws_bytes, device=dev, dtype=torch.uint8)
+    out = torch.empty(T, d, device=dev, dtype=torch.bfloat16)
+    side = fork = join = None
+    if overlap:
+        fork_ev, join_ev = side_events(dev)
+        side, fork, join = side_stream(dev).cuda_stream, fork_ev.cuda_event, join_ev.cuda_event
+    L.call("hmoe_moe_block", L.ptr(x), x.stride(0), L.ptr(gate_w), L.ptr(gate_b), n_group, topk_group, float(scaling),
+           L.ptr(wgu), L.ptr(wgu_s), L.dt(wgu_s) if wgu_s is not None else 0, L.ptr(wd), L.ptr(wd_s),
+           L.dt(wd_s) if wd_s is not None else 0, w_dt, L.ptr(sh_wgu), L.ptr(sh_wd), L.ptr(sh_count), sh, T, d, E, k, h,
+           L.ptr(out), L.ptr(ws), ws_bytes, _dev_stream(x), side, fork, join)
+    return out
 
 
 def route_sigmoid_group(x: torch.Tensor, wr: torch.Tensor, k: int, n_group: int, topk_group: int, expert_bias=None,

@@ -160,6 +160,11 @@ class PoziomkaMoE(nn.Module):
         T, k, E = x2.shape[0], self.top_k, self._wgu.shape[0]
         gw, gb = self._gate_tensors()
         wgu_sh, wd_sh = self.shared_experts._stack.get(self.shared_experts)
+        if T > 0 and ops.probe is None:
+            return ops.moe_block(x2, gw, gb, k, self.n_group, self.topk_group, self.scaling, self._wgu, self._wgu_s,
+                                 self._wd, self._wd_s, wgu_sh, wd_sh, _one_count(T, x2.device),
+                                 overlap=self.overlap_shared).view(shape)
+        # event timing of single ops (bench.py's probe) needs the launches apart: the same entry points one by one
         side = ops.side_stream(x2.device) if self.overlap_shared and T > 0 else None
         if side is not None:  # fork: the shared expert needs only x
             main = torch.cuda.current_stream(x2.device)
