@@ -36,6 +36,7 @@ struct RowOffs {
 // The kernel
 // ----------------------------------------------------------------------------------------------------------------
 // A_BLK: the A rows (MGROUP) come from the row-group tiles of the sorted rows (gemm_common.h), not from A's rows.
+// With EPI_STORE: from act in blocked rows (gemm_common.h), as EPI_SWIGLU stores them with p.c_blocked.
 // F16: the 16-bit operands, row scales and outputs are fp16 (v_mfma_f32_32x32x16_f16) instead of bf16; forward
 // epilogues (store, SwiGLU) only.
 template <class C, int MODE, bool A_MN, bool B_MN, int EPI, bool A_BLK = false, bool F16 = false>
@@ -45,7 +46,8 @@ __global__ __launch_bounds__(C::NT, 1) void grouped_gemm_kernel(GemmParams p) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   __shared__ int s_rstart[kMaxEGemm + 1];  // row starts (M < 2^31: checked on the host)
   __shared__ int s_tstart[kMaxEGemm + 1];  // MGROUP: prefix of ceil(count / BM); KGROUP: one m-tile per expert
-  __shared__ int s_gstart[A_BLK ? kMaxEGemm + 1 : 1];  // A_BLK: prefix of ceil(count / 128) (row groups)
+  constexpr bool A_ROWBLK = A_BLK && EPI == EPI_STORE, A_GROUPS = A_BLK && !A_ROWBLK;
+  __shared__ int s_gstart[A_GROUPS ? kMaxEGemm + 1 : 1];  // row-group tiles: prefix of ceil(count / 128)
   // per-row epilogue inputs of the tile (scatter index, routing weight), double-buffered by tile parity: a wave
   // that has finished its epilogue may already fill the next tile's while others still read this one.  The copy
   // starts at the 16-byte boundary below row0 (up to 7 leading 2-byte elements) and writes whole 1 KB blocks: one
@@ -75,7 +77,7 @@ __global__ __launch_bounds__(C::NT, 1) void grouped_gemm_kernel(GemmParams p) {
         c = c < 0 ? 0 : (c > p.M ? p.M : c);  // garbage counts must not blow up the tile loop
         rs += c;
         ts += MODE == MGROUP ? (int)((c + C::BM - 1) / C::BM) : 1;
-        if constexpr (A_BLK) gs += (int)((c + kTileGroupRows - 1) / kTileGroupRows);
+        if constexpr (A_GROUPS) gs += (int)((c + kTileGroupRows - 1) / kTileGroupRows);
       }
     }
     int64_t irs = rs;
@@ -102,7 +104,7 @@ __global__ __launch_bounds__(C::NT, 1) void grouped_gemm_kernel(GemmParams p) {
         s_tstart[e] = t0;
         r0 += c;
         t0 += MODE == MGROUP ? (int)((c + C::BM - 1) / C::BM) : 1;
-        if constexpr (A_BLK) {
+        if constexpr (A_GROUPS) {
           s_gstart[e] = g0;
           g0 += (int)((c + kTileGroupRows - 1) / kTileGroupRows);
         }
@@ -227,7 +229,21 @@ __global__ __launch_bounds__(C::NT, 1) void grouped_gemm_kernel(GemmParams p) {
     if constexpr (MODE == MGROUP) {
       static_assert(!A_MN, "MGROUP A is K-contiguous");
       ta.K = kvalid;
-      if constexpr (A_BLK) {
+      if constexpr (A_ROWBLK) {
+        ta.kmul = kTileSliceBytes / kBK;
+        ta.rsrc = make_rsrc(p.A);
+        const int64_t nsl = (p.K + kBK - 1) / kBK;
+#pragma unroll
+        for (int i = 0; i < ta.PER_WAVE; ++i) {
+          const int rr = ta.row_of(wave, lane, i);
+          const int64_t r = row0 + rr;
+          const int c = (lane & 3) ^ swz_k(rr);
+          ta.voff[i] = r < row_end ? (uint32_t)(r / kTileGroupRows * nsl * kTileSliceBytes +
+                                                r % kTileGroupRows * (2 * kBK) + c * 16)
+                                   : kOOB;
+          ta.chunk[i] = c;
+        }
+      } else if constexpr (A_BLK) {
         // row-group tiles: instruction I's 16 rows (tile rows 16 I ..) are one 1 KB run of their group's slice
         ta.kmul = kTileSliceBytes / kBK;
         ta.rsrc = make_rsrc(p.A);
@@ -706,8 +722,13 @@ __global__ __launch_bounds__(C::NT, 1) void grouped_gemm_kernel(GemmParams p) {
     // are issued before their stores, so a pass waits for LDS once per sub-plane pair, not once per store.
     // PAIRED false: each piece's read just ahead of its store instead (what the bf16 forward epilogues measured
     // fastest, by 1%)
+    // blocked_tag: blocked rows (rows.o points at a row's part of its block's first k-slice)
     auto drain_rows = [&](auto nsp_tag, int sp0, int rowbytes, int es, char* base, const RowOffs rows, int ncols,
-                          auto paired_tag) {
+                          auto paired_tag, auto blocked_tag) {
+      auto col_off = [&](int n) -> int64_t {
+        if constexpr (decltype(blocked_tag)::value) return (int64_t)(n / kBK) * kTileSliceBytes + n % kBK * 2;
+        return (int64_t)n * es;
+      };
       constexpr int NSPX = decltype(nsp_tag)::value;
       constexpr bool PAIRED = decltype(paired_tag)::value;
       const int c = lane & 7;
@@ -722,7 +743,7 @@ __global__ __launch_bounds__(C::NT, 1) void grouped_gemm_kernel(GemmParams p) {
         const bool cok = sp * 128 + c * 16 < rowbytes && n < ncols;  // a narrow array fills part of a sub-plane
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          if (cok && rows.o[j] >= 0) *reinterpret_cast<uint4*>(base + rows.o[j] + (int64_t)n * es) = v[j];
+          if (cok && rows.o[j] >= 0) *reinterpret_cast<uint4*>(base + rows.o[j] + col_off(n)) = v[j];
       };
       if constexpr (PAIRED) {
 #pragma unroll
@@ -747,7 +768,7 @@ __global__ __launch_bounds__(C::NT, 1) void grouped_gemm_kernel(GemmParams p) {
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
             const uint4 v = *reinterpret_cast<const uint4*>(sp_addr(sp0 + sp, 8 * j + (lane >> 3), c * 16));
-            if (cok && rows.o[j] >= 0) *reinterpret_cast<uint4*>(base + rows.o[j] + (int64_t)n * es) = v;
+            if (cok && rows.o[j] >= 0) *reinterpret_cast<uint4*>(base + rows.o[j] + col_off(n)) = v;
           }
         }
       }
@@ -799,11 +820,11 @@ __global__ __launch_bounds__(C::NT, 1) void grouped_gemm_kernel(GemmParams p) {
         if (p.c_f32) {
           park_all(std::true_type{});
           drain_rows(std::integral_constant<int, C::FN * 32 * 4 / 128>{}, 0, C::FN * 32 * 4, 4, base, rows, p.N,
-                     std::true_type{});
+                     std::true_type{}, std::false_type{});
         } else {
           park_all(std::false_type{});
           drain_rows(std::integral_constant<int, C::FN * 32 * 2 / 128>{}, 0, C::FN * 32 * 2, 2, base, rows, p.N,
-                     std::true_type{});
+                     std::true_type{}, std::false_type{});
         }
       } else if constexpr (EPI == EPI_STORE || EPI == EPI_STORE_F32) {
         constexpr int ES = EPI == EPI_STORE_F32 ? 4 : 2;
@@ -850,12 +871,13 @@ __global__ __launch_bounds__(C::NT, 1) void grouped_gemm_kernel(GemmParams p) {
         });
         constexpr std::bool_constant<C::BE == 1> paired{};  // int8 weights: paired reads (bf16: one by one)
         drain_rows(std::integral_constant<int, NSP>{}, 0, RB, ES,
-                   reinterpret_cast<char*>(p.C) + (EPI == EPI_STORE_F32 ? part * p.M * p.ldc * ES : 0), rows, p.N, paired);
+                   reinterpret_cast<char*>(p.C) + (EPI == EPI_STORE_F32 ? part * p.M * p.ldc * ES : 0), rows, p.N, paired,
+                   std::false_type{});
         if constexpr (C::BE == 2) {
           if (aux)
             drain_rows(std::integral_constant<int, (C::FN * 32 * 2 + 127) / 128>{}, NSP, C::FN * 32 * 2, 2,
                        reinterpret_cast<char*>(p.aux),
-                       rows_of(rbase, [&](int, int64_t row) { return row * p.ldc * 2; }), p.N, paired);
+                       rows_of(rbase, [&](int, int64_t row) { return row * p.ldc * 2; }), p.N, paired, std::false_type{});
         }
       } else if constexpr (EPI == EPI_SWIGLU) {
         // fragments b < FN/2 hold gate columns, b + FN/2 the matching up columns (tile columns + BN/2); the wave's
@@ -910,15 +932,23 @@ __global__ __launch_bounds__(C::NT, 1) void grouped_gemm_kernel(GemmParams p) {
         else
           park_all(aux, std::false_type{});
         constexpr std::bool_constant<C::BE == 1> paired{};  // int8 weights: paired reads (bf16: one by one)
-        drain_rows(std::integral_constant<int, NSP>{}, 0, RB, 2, reinterpret_cast<char*>(p.C),
-                   rows_of(rbase, [&](int, int64_t row) { return row * p.ldc * 2; }), p.N, paired);
+        if (p.c_blocked) {
+          const int64_t block_bytes = (int64_t)((p.N + kBK - 1) / kBK) * kTileSliceBytes;
+          drain_rows(std::integral_constant<int, NSP>{}, 0, RB, 2, reinterpret_cast<char*>(p.C),
+                     rows_of(rbase, [&](int, int64_t row) {
+                       return row / kTileGroupRows * block_bytes + row % kTileGroupRows * (2 * kBK);
+                     }), p.N, paired, std::true_type{});
+        } else {
+          drain_rows(std::integral_constant<int, NSP>{}, 0, RB, 2, reinterpret_cast<char*>(p.C),
+                     rows_of(rbase, [&](int, int64_t row) { return row * p.ldc * 2; }), p.N, paired, std::false_type{});
+        }
         if constexpr (C::BE == 2) {
           if (aux) {
             const RowOffs rows = rows_of(rbase, [&](int, int64_t row) { return row * (int64_t)(2 * p.h) * 2; });
             drain_rows(std::integral_constant<int, NSP>{}, NSP, RB, 2, reinterpret_cast<char*>(p.aux), rows, p.N,
-                       paired);
+                       paired, std::false_type{});
             drain_rows(std::integral_constant<int, NSP>{}, 2 * NSP, RB, 2, reinterpret_cast<char*>(p.aux + p.h), rows,
-                       p.N, paired);
+                       p.N, paired, std::false_type{});
           }
         }
       } else if constexpr (EPI == EPI_SWIGLU_BWD) {
@@ -1166,8 +1196,8 @@ static FewTile pick_few(int64_t M, int64_t E, int64_t ncols, int64_t K, bool int
 // launches the few-rows kernel if the rule picks it: *done, and the launch's status
 template <int EPI, bool F16, int BE>
 static int launch_few(const GemmParams& p, int64_t ncols, hipStream_t s, bool* done) {
-  // (a [g | u] or unscaled copy is the persistent kernel's)
-  const FewTile t = p.aux ? FEW_NONE : pick_few<EPI>(p.M, p.E, ncols, p.K, BE == 1);
+  // (a [g | u] or unscaled copy and act in blocked rows are the persistent kernel's)
+  const FewTile t = p.aux || p.c_blocked ? FEW_NONE : pick_few<EPI>(p.M, p.E, ncols, p.K, BE == 1);
   *done = t != FEW_NONE;
   switch (t) {
     case FEW_32x128: return launch_few_tile<FewCfg<1, 2, 4, BE>, EPI, F16>(p, ncols, s);
@@ -1190,18 +1220,20 @@ static int launch_fwd(const GemmParams& p, int64_t ncols, bool f16, hipStream_t 
 }
 
 // int8 weights: the int8 tile configurations
-template <int EPI, bool F16 = false>
+template <int EPI, bool F16, bool A_BLK>
 static int launch_mgroup_i8_t(const GemmParams& p, int64_t ncols, hipStream_t s) {
-  bool done;
-  const int rc = launch_few<EPI, F16, 1>(p, ncols, s, &done);
-  if (done) return rc;
+  if constexpr (!A_BLK) {
+    bool done;
+    const int rc = launch_few<EPI, F16, 1>(p, ncols, s, &done);
+    if (done) return rc;
+  }
   const int64_t tl = mgroup_tiles<CfgL8, EPI>(p.M, p.E, ncols);
-  if (pick_large_mgroup<EPI>(tl, ncols)) return launch<CfgL8, MGROUP, false, true, EPI, false, F16>(p, tl, s);
-  return launch<CfgS8, MGROUP, false, true, EPI, false, F16>(p, mgroup_tiles<CfgS8, EPI>(p.M, p.E, ncols), s);
+  if (pick_large_mgroup<EPI>(tl, ncols)) return launch<CfgL8, MGROUP, false, true, EPI, A_BLK, F16>(p, tl, s);
+  return launch<CfgS8, MGROUP, false, true, EPI, A_BLK, F16>(p, mgroup_tiles<CfgS8, EPI>(p.M, p.E, ncols), s);
 }
-template <int EPI>
+template <int EPI, bool A_BLK = false>
 static int launch_mgroup_i8(const GemmParams& p, int64_t ncols, bool f16, hipStream_t s) {
-  return f16 ? launch_mgroup_i8_t<EPI, true>(p, ncols, s) : launch_mgroup_i8_t<EPI, false>(p, ncols, s);
+  return f16 ? launch_mgroup_i8_t<EPI, true, A_BLK>(p, ncols, s) : launch_mgroup_i8_t<EPI, false, A_BLK>(p, ncols, s);
 }
 
 // activation element type of the forward entry points: bf16 or fp16 (rc: HMOE_OK or HMOE_ERR_DTYPE)
@@ -1257,6 +1289,166 @@ static int check_common(const void* counts, int counts_dtype, int64_t E, int64_t
   return HMOE_OK;
 }
 
+// ---- the forward entry points; act_blocked: act (M, h) is written and read in blocked rows ----
+bool act_blocked_rule(int64_t M, int64_t E, int64_t d, int64_t h, bool int8) {
+  return off32(blocked_bytes(M, h)) && pick_few<EPI_SWIGLU>(M, E, h, d, int8) == FEW_NONE &&
+         pick_few<EPI_STORE>(M, E, d, h, int8) == FEW_NONE;
+}
+
+int gate_up_swiglu_at(const void* x, int64_t ldx, const int32_t* a_idx, const void* wgu, int64_t E, int64_t d, int64_t
+                      h, const void* counts, int counts_dtype, int64_t M, void* act, void* gu, int dtype,
+                      hmoe_stream_t stream, bool act_blocked) {
+  int rc = check_common(counts, counts_dtype, E, M);
+  if (rc) return rc;
+  const bool f16 = act16(dtype, &rc);
+  if (rc) return rc;
+  if (M == 0) return HMOE_OK;
+  if (!x || !wgu || !act || d <= 0 || h <= 0) return HMOE_ERR_ARG;
+  if (d % 8 || h % 8 || ldx % 8 || ldx < d) return HMOE_ERR_SHAPE;
+  if (!al16(x) || !al16(wgu) || !al16(act) || !al16(gu)) return HMOE_ERR_ARG;
+  if ((a_idx && !off32(M * ldx * 2)) || !off32(d * 2 * h * 2)) return HMOE_ERR_SHAPE;
+  GemmParams p = base_params(counts, counts_dtype, E, M);
+  p.A = static_cast<const uint16_t*>(x);
+  p.lda = ldx;
+  p.a_idx = a_idx;
+  p.B = (wgu);
+  p.ldb = 2 * h;
+  p.strideBe = d * 2 * h;
+  p.K = (int)d;
+  p.N = (int)h;
+  p.h = (int)h;
+  p.C = act;
+  p.ldc = h;
+  p.c_blocked = act_blocked;
+  p.aux = static_cast<uint16_t*>(gu);
+  return launch_fwd<EPI_SWIGLU>(p, h, f16, reinterpret_cast<hipStream_t>(stream));
+}
+
+int gate_up_swiglu_tiles_at(const void* xs_tiles, const void* wgu, int64_t E, int64_t d, int64_t h, const void*
+                            counts, int counts_dtype, int64_t M, void* act, void* gu, int dtype, hmoe_stream_t stream,
+                            bool act_blocked) {
+  int rc = check_common(counts, counts_dtype, E, M);
+  if (rc) return rc;
+  const bool f16 = act16(dtype, &rc);
+  if (rc) return rc;
+  if (M == 0) return HMOE_OK;
+  if (!xs_tiles || !wgu || !act || d <= 0 || h <= 0) return HMOE_ERR_ARG;
+  if (d % 8 || h % 8) return HMOE_ERR_SHAPE;
+  if (!al16(xs_tiles) || !al16(wgu) || !al16(act) || !al16(gu)) return HMOE_ERR_ARG;
+  if (!off32(tiles_bytes(M, E, d)) || !off32(d * 2 * h * 2)) return HMOE_ERR_SHAPE;
+  GemmParams p = base_params(counts, counts_dtype, E, M);
+  p.A = static_cast<const uint16_t*>(xs_tiles);
+  p.lda = d;
+  p.B = (wgu);
+  p.ldb = 2 * h;
+  p.strideBe = d * 2 * h;
+  p.K = (int)d;
+  p.N = (int)h;
+  p.h = (int)h;
+  p.C = act;
+  p.ldc = h;
+  p.c_blocked = act_blocked;
+  p.aux = static_cast<uint16_t*>(gu);
+  return launch_fwd<EPI_SWIGLU, true>(p, h, f16, reinterpret_cast<hipStream_t>(stream));
+}
+
+int down_scatter_at(const void* act, const void* wd, int64_t E, int64_t h, int64_t d, const void* counts, int
+                    counts_dtype, int64_t M, const uint16_t* w_sorted, const int32_t* y_idx, void* y, void* yhat, int
+                    dtype, hmoe_stream_t stream, bool act_blocked) {
+  int rc = check_common(counts, counts_dtype, E, M);
+  if (rc) return rc;
+  const bool f16 = act16(dtype, &rc);
+  if (rc) return rc;
+  if (M == 0) return HMOE_OK;
+  if (!act || !wd || !y || d <= 0 || h <= 0) return HMOE_ERR_ARG;
+  if (d % 8 || h % 8) return HMOE_ERR_SHAPE;
+  if (!al16(act) || !al16(wd) || !al16(y) || !al16(yhat)) return HMOE_ERR_ARG;
+  if (!off32(h * d * 2)) return HMOE_ERR_SHAPE;
+  if (act_blocked && !off32(blocked_bytes(M, h))) return HMOE_ERR_SHAPE;
+  GemmParams p = base_params(counts, counts_dtype, E, M);
+  p.A = static_cast<const uint16_t*>(act);
+  p.lda = h;
+  p.B = (wd);
+  p.ldb = d;
+  p.strideBe = h * d;
+  p.K = (int)h;
+  p.N = (int)d;
+  p.C = y;
+  p.ldc = d;
+  p.y_idx = y_idx;
+  p.scale = w_sorted;
+  p.scale_f32 = 0;
+  p.aux = static_cast<uint16_t*>(yhat);
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  return act_blocked ? launch_fwd<EPI_STORE, true>(p, d, f16, s) : launch_fwd<EPI_STORE>(p, d, f16, s);
+}
+
+int gate_up_swiglu_i8_at(const void* x, int64_t ldx, const int32_t* a_idx, const void* wgu_q, const void* wgu_s, int
+                         wgu_s_dtype, int64_t E, int64_t d, int64_t h, const void* counts, int counts_dtype, int64_t
+                         M, void* act, int dtype, hmoe_stream_t stream, bool act_blocked) {
+  int rc = check_common(counts, counts_dtype, E, M);
+  if (rc) return rc;
+  const bool f16 = act16(dtype, &rc);
+  if (rc) return rc;
+  if (M == 0) return HMOE_OK;
+  if (!x || !act || d <= 0 || h <= 0) return HMOE_ERR_ARG;
+  if (d % 8 || h % 16 || ldx % 8 || ldx < d) return HMOE_ERR_SHAPE;
+  if (!al16(x) || !al16(act)) return HMOE_ERR_ARG;
+  if ((a_idx && !off32(M * ldx * 2)) || !off32(d * 2 * h)) return HMOE_ERR_SHAPE;
+  if ((rc = check_i8(wgu_q, 2 * h, d, 2 * h, d * 2 * h, wgu_s, wgu_s_dtype))) return rc;
+  GemmParams p = base_params(counts, counts_dtype, E, M);
+  p.A = static_cast<const uint16_t*>(x);
+  p.lda = ldx;
+  p.a_idx = a_idx;
+  p.B = wgu_q;
+  p.ldb = 2 * h;
+  p.strideBe = d * 2 * h;
+  p.K = (int)d;
+  p.N = (int)h;
+  p.h = (int)h;
+  p.C = act;
+  p.ldc = h;
+  p.c_blocked = act_blocked;
+  p.w_scale = wgu_s;
+  p.w_scale_f32 = wgu_s_dtype == HMOE_DT_F32;
+  p.ldws = 2 * h;
+  return launch_mgroup_i8<EPI_SWIGLU>(p, h, f16, reinterpret_cast<hipStream_t>(stream));
+}
+
+int down_scatter_i8_at(const void* act, const void* wd_q, const void* wd_s, int wd_s_dtype, int64_t E, int64_t h,
+                       int64_t d, const void* counts, int counts_dtype, int64_t M, const uint16_t* w_sorted, const
+                       int32_t* y_idx, void* y, int dtype, hmoe_stream_t stream, bool act_blocked) {
+  int rc = check_common(counts, counts_dtype, E, M);
+  if (rc) return rc;
+  const bool f16 = act16(dtype, &rc);
+  if (rc) return rc;
+  if (M == 0) return HMOE_OK;
+  if (!act || !y || d <= 0 || h <= 0) return HMOE_ERR_ARG;
+  if (h % 8 || d % 16) return HMOE_ERR_SHAPE;
+  if (!al16(act) || !al16(y)) return HMOE_ERR_ARG;
+  if (!off32(h * d)) return HMOE_ERR_SHAPE;
+  if (act_blocked && !off32(blocked_bytes(M, h))) return HMOE_ERR_SHAPE;
+  if ((rc = check_i8(wd_q, d, h, d, h * d, wd_s, wd_s_dtype))) return rc;
+  GemmParams p = base_params(counts, counts_dtype, E, M);
+  p.A = static_cast<const uint16_t*>(act);
+  p.lda = h;
+  p.B = wd_q;
+  p.ldb = d;
+  p.strideBe = h * d;
+  p.K = (int)h;
+  p.N = (int)d;
+  p.C = y;
+  p.ldc = d;
+  p.y_idx = y_idx;
+  p.scale = w_sorted;
+  p.scale_f32 = 0;
+  p.w_scale = wd_s;
+  p.w_scale_f32 = wd_s_dtype == HMOE_DT_F32;
+  p.ldws = d;
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  return act_blocked ? launch_mgroup_i8<EPI_STORE, true>(p, d, f16, s) : launch_mgroup_i8<EPI_STORE>(p, d, f16, s);
+}
+
 }  // namespace hmoe
 
 using namespace hmoe;
@@ -1310,148 +1502,31 @@ int hmoe_grouped_mm(const void* a, int64_t lda, int a_dtype, const void* w, int 
 int hmoe_gate_up_swiglu(const void* x, int64_t ldx, const int32_t* a_idx, const void* wgu, int64_t E, int64_t d,
                         int64_t h, const void* counts, int counts_dtype, int64_t M, void* act, void* gu, int dtype,
                         hmoe_stream_t stream) {
-  int rc = check_common(counts, counts_dtype, E, M);
-  if (rc) return rc;
-  const bool f16 = act16(dtype, &rc);
-  if (rc) return rc;
-  if (M == 0) return HMOE_OK;
-  if (!x || !wgu || !act || d <= 0 || h <= 0) return HMOE_ERR_ARG;
-  if (d % 8 || h % 8 || ldx % 8 || ldx < d) return HMOE_ERR_SHAPE;
-  if (!al16(x) || !al16(wgu) || !al16(act) || !al16(gu)) return HMOE_ERR_ARG;
-  if ((a_idx && !off32(M * ldx * 2)) || !off32(d * 2 * h * 2)) return HMOE_ERR_SHAPE;
-  GemmParams p = base_params(counts, counts_dtype, E, M);
-  p.A = static_cast<const uint16_t*>(x);
-  p.lda = ldx;
-  p.a_idx = a_idx;
-  p.B = (wgu);
-  p.ldb = 2 * h;
-  p.strideBe = d * 2 * h;
-  p.K = (int)d;
-  p.N = (int)h;
-  p.h = (int)h;
-  p.C = act;
-  p.ldc = h;
-  p.aux = static_cast<uint16_t*>(gu);
-  return launch_fwd<EPI_SWIGLU>(p, h, f16, reinterpret_cast<hipStream_t>(stream));
+  return gate_up_swiglu_at(x, ldx, a_idx, wgu, E, d, h, counts, counts_dtype, M, act, gu, dtype, stream, false);
 }
 
 int hmoe_gate_up_swiglu_tiles(const void* xs_tiles, const void* wgu, int64_t E, int64_t d, int64_t h,
                               const void* counts, int counts_dtype, int64_t M, void* act, void* gu, int dtype,
                               hmoe_stream_t stream) {
-  int rc = check_common(counts, counts_dtype, E, M);
-  if (rc) return rc;
-  const bool f16 = act16(dtype, &rc);
-  if (rc) return rc;
-  if (M == 0) return HMOE_OK;
-  if (!xs_tiles || !wgu || !act || d <= 0 || h <= 0) return HMOE_ERR_ARG;
-  if (d % 8 || h % 8) return HMOE_ERR_SHAPE;
-  if (!al16(xs_tiles) || !al16(wgu) || !al16(act) || !al16(gu)) return HMOE_ERR_ARG;
-  if (!off32(tiles_bytes(M, E, d)) || !off32(d * 2 * h * 2)) return HMOE_ERR_SHAPE;
-  GemmParams p = base_params(counts, counts_dtype, E, M);
-  p.A = static_cast<const uint16_t*>(xs_tiles);
-  p.lda = d;
-  p.B = (wgu);
-  p.ldb = 2 * h;
-  p.strideBe = d * 2 * h;
-  p.K = (int)d;
-  p.N = (int)h;
-  p.h = (int)h;
-  p.C = act;
-  p.ldc = h;
-  p.aux = static_cast<uint16_t*>(gu);
-  return launch_fwd<EPI_SWIGLU, true>(p, h, f16, reinterpret_cast<hipStream_t>(stream));
+  return gate_up_swiglu_tiles_at(xs_tiles, wgu, E, d, h, counts, counts_dtype, M, act, gu, dtype, stream, false);
 }
 
 int hmoe_down_scatter(const void* act, const void* wd, int64_t E, int64_t h, int64_t d, const void* counts,
                       int counts_dtype, int64_t M, const uint16_t* w_sorted, const int32_t* y_idx, void* y,
                       void* yhat, int dtype, hmoe_stream_t stream) {
-  int rc = check_common(counts, counts_dtype, E, M);
-  if (rc) return rc;
-  const bool f16 = act16(dtype, &rc);
-  if (rc) return rc;
-  if (M == 0) return HMOE_OK;
-  if (!act || !wd || !y || d <= 0 || h <= 0) return HMOE_ERR_ARG;
-  if (d % 8 || h % 8) return HMOE_ERR_SHAPE;
-  if (!al16(act) || !al16(wd) || !al16(y) || !al16(yhat)) return HMOE_ERR_ARG;
-  if (!off32(h * d * 2)) return HMOE_ERR_SHAPE;
-  GemmParams p = base_params(counts, counts_dtype, E, M);
-  p.A = static_cast<const uint16_t*>(act);
-  p.lda = h;
-  p.B = (wd);
-  p.ldb = d;
-  p.strideBe = h * d;
-  p.K = (int)h;
-  p.N = (int)d;
-  p.C = y;
-  p.ldc = d;
-  p.y_idx = y_idx;
-  p.scale = w_sorted;
-  p.scale_f32 = 0;
-  p.aux = static_cast<uint16_t*>(yhat);
-  return launch_fwd<EPI_STORE>(p, d, f16, reinterpret_cast<hipStream_t>(stream));
+  return down_scatter_at(act, wd, E, h, d, counts, counts_dtype, M, w_sorted, y_idx, y, yhat, dtype, stream, false);
 }
 
 int hmoe_gate_up_swiglu_i8(const void* x, int64_t ldx, const int32_t* a_idx, const void* wgu_q, const void* wgu_s,
                            int wgu_s_dtype, int64_t E, int64_t d, int64_t h, const void* counts, int counts_dtype,
                            int64_t M, void* act, int dtype, hmoe_stream_t stream) {
-  int rc = check_common(counts, counts_dtype, E, M);
-  if (rc) return rc;
-  const bool f16 = act16(dtype, &rc);
-  if (rc) return rc;
-  if (M == 0) return HMOE_OK;
-  if (!x || !act || d <= 0 || h <= 0) return HMOE_ERR_ARG;
-  if (d % 8 || h % 16 || ldx % 8 || ldx < d) return HMOE_ERR_SHAPE;
-  if (!al16(x) || !al16(act)) return HMOE_ERR_ARG;
-  if ((a_idx && !off32(M * ldx * 2)) || !off32(d * 2 * h)) return HMOE_ERR_SHAPE;
-  if ((rc = check_i8(wgu_q, 2 * h, d, 2 * h, d * 2 * h, wgu_s, wgu_s_dtype))) return rc;
-  GemmParams p = base_params(counts, counts_dtype, E, M);
-  p.A = static_cast<const uint16_t*>(x);
-  p.lda = ldx;
-  p.a_idx = a_idx;
-  p.B = wgu_q;
-  p.ldb = 2 * h;
-  p.strideBe = d * 2 * h;
-  p.K = (int)d;
-  p.N = (int)h;
-  p.h = (int)h;
-  p.C = act;
-  p.ldc = h;
-  p.w_scale = wgu_s;
-  p.w_scale_f32 = wgu_s_dtype == HMOE_DT_F32;
-  p.ldws = 2 * h;
-  return launch_mgroup_i8<EPI_SWIGLU>(p, h, f16, reinterpret_cast<hipStream_t>(stream));
+  return gate_up_swiglu_i8_at(x, ldx, a_idx, wgu_q, wgu_s, wgu_s_dtype, E, d, h, counts, counts_dtype, M, act, dtype, stream, false);
 }
 
 int hmoe_down_scatter_i8(const void* act, const void* wd_q, const void* wd_s, int wd_s_dtype, int64_t E, int64_t h,
                          int64_t d, const void* counts, int counts_dtype, int64_t M, const uint16_t* w_sorted,
                          const int32_t* y_idx, void* y, int dtype, hmoe_stream_t stream) {
-  int rc = check_common(counts, counts_dtype, E, M);
-  if (rc) return rc;
-  const bool f16 = act16(dtype, &rc);
-  if (rc) return rc;
-  if (M == 0) return HMOE_OK;
-  if (!act || !y || d <= 0 || h <= 0) return HMOE_ERR_ARG;
-  if (h % 8 || d % 16) return HMOE_ERR_SHAPE;
-  if (!al16(act) || !al16(y)) return HMOE_ERR_ARG;
-  if (!off32(h * d)) return HMOE_ERR_SHAPE;
-  if ((rc = check_i8(wd_q, d, h, d, h * d, wd_s, wd_s_dtype))) return rc;
-  GemmParams p = base_params(counts, counts_dtype, E, M);
-  p.A = static_cast<const uint16_t*>(act);
-  p.lda = h;
-  p.B = wd_q;
-  p.ldb = d;
-  p.strideBe = h * d;
-  p.K = (int)h;
-  p.N = (int)d;
-  p.C = y;
-  p.ldc = d;
-  p.y_idx = y_idx;
-  p.scale = w_sorted;
-  p.scale_f32 = 0;
-  p.w_scale = wd_s;
-  p.w_scale_f32 = wd_s_dtype == HMOE_DT_F32;
-  p.ldws = d;
-  return launch_mgroup_i8<EPI_STORE>(p, d, f16, reinterpret_cast<hipStream_t>(stream));
+  return down_scatter_i8_at(act, wd_q, wd_s, wd_s_dtype, E, h, d, counts, counts_dtype, M, w_sorted, y_idx, y, dtype, stream, false);
 }
 
 // Checks and parameters shared by the two down-dgrad entry points (rc: HMOE_OK, or the error to return).

@@ -37,6 +37,11 @@ struct Cfg {
 // uses bits 2-3 of the row only, so any 16-row run of a group is a valid piece of a tile's image).
 static_assert(kTileK == kBK, "row-group tiles hold one LDS slice per 32 k");
 constexpr int kTileSliceBytes = kTileGroupRows * kBK * 2;
+// Blocked rows (act between the forward GEMMs): blocks of 128 sorted rows whatever their experts, each k-slice by k-slice
+// like a row group but with a row's 64 bytes in order: row r, column c of a matrix of K columns at byte
+// (r / 128 * nslices + c / 32) * 8 KB + r % 128 * 64 + c % 32 * 2.  A copy of 16 rows reads 1 KB in a run here too (9
+// lines where an expert starts at an odd row), and unlike row groups blocked rows take no more memory than the matrix
+// (up to whole blocks and slices).
 
 // ----------------------------------------------------------------------------------------------------------------
 // LDS tile layouts (one k-slice of BK = 32)
@@ -385,6 +390,7 @@ struct GemmParams {
   // epilogue
   void* C;  // EPI_STORE: y; EPI_SWIGLU: act (M, h); EPI_SWIGLU_BWD: dgu (M, 2h); EPI_WGRAD: dw (E, P, N)
   int64_t ldc, strideCe;
+  int c_blocked;            // EPI_SWIGLU: act in blocked rows
   int c_f32;                // EPI_WGRAD / EPI_STORE: fp32 output
   const int32_t* y_idx;     // EPI_STORE scatter
   const void* scale;        // EPI_STORE / EPI_SWIGLU_BWD per-row scale: fp32, or the activations' 16-bit type

@@ -4,9 +4,7 @@
 // are called one by one, so the outputs are identical; what the one call removes is the host work between them (a
 // binding's per-call argument checks, output allocations and calls), which bounds small layers: a 512-token layer
 // takes about 43 us of GPU time and about 80 us of host time when driven op by op from Python.
-#include "../../include/hmoe.h"
-
-#include <hip/hip_runtime.h>
+#include "hmoe_common.h"
 
 #include <cstddef>
 #include <cstdint>
@@ -20,10 +18,16 @@ constexpr int64_t kTilesMinH = 4096;
 
 size_t al256(size_t v) { return (v + 255) & ~static_cast<size_t>(255); }
 
+// act between the two GEMMs: bytes as rows or in blocked rows
+size_t act_bytes(int64_t M, int64_t h, bool blocked) {
+  return blocked ? static_cast<size_t>(hmoe::blocked_bytes(M, h))
+                 : static_cast<size_t>(M) * static_cast<size_t>(h) * 2;
+}
+
 struct FwdLayout {
   size_t logits, counts, starts, order, a_idx, inv, w_sorted, n_invalid, dws, tiles, act, y, total;
   size_t dws_bytes;
-  bool tiles_on;
+  bool tiles_on, act_blocked;
 };
 
 // Byte offsets of the intermediates; false for sizes no entry point accepts.
@@ -49,7 +53,8 @@ bool fwd_layout(int64_t T, int64_t d, int E, int k, int64_t h, FwdLayout& L) {
   L.n_invalid = take(4);
   L.dws = take(L.dws_bytes);
   L.tiles = L.tiles_on ? take(tiles_bytes) : 0;
-  L.act = take(static_cast<size_t>(M) * static_cast<size_t>(h) * 2);
+  L.act_blocked = hmoe::act_blocked_rule(M, E, d, h, false);
+  L.act = take(act_bytes(M, h, L.act_blocked));
   L.y = take(static_cast<size_t>(M) * static_cast<size_t>(d) * 2);
   L.total = o;
   return true;
@@ -101,13 +106,14 @@ int hmoe_moe_forward(const void* x, int64_t ldx, const void* wr, const float* bi
                            a_idx, inv, w_sorted, n_invalid, ws + L.dws, L.dws_bytes, HMOE_DT_BF16, stream);
   if (rc != HMOE_OK) return rc;
   if (L.tiles_on)
-    rc = hmoe_gate_up_swiglu_tiles(tiles, wgu, E, d, h, counts, HMOE_DT_I32, M, act, nullptr, HMOE_DT_BF16, stream);
+    rc = hmoe::gate_up_swiglu_tiles_at(tiles, wgu, E, d, h, counts, HMOE_DT_I32, M, act, nullptr, HMOE_DT_BF16, stream,
+                                       L.act_blocked);
   else
-    rc = hmoe_gate_up_swiglu(x, ldx, a_idx, wgu, E, d, h, counts, HMOE_DT_I32, M, act, nullptr, HMOE_DT_BF16,
-                             stream);
+    rc = hmoe::gate_up_swiglu_at(x, ldx, a_idx, wgu, E, d, h, counts, HMOE_DT_I32, M, act, nullptr, HMOE_DT_BF16,
+                                 stream, L.act_blocked);
   if (rc != HMOE_OK) return rc;
-  rc = hmoe_down_scatter(act, wd, E, h, d, counts, HMOE_DT_I32, M, w_sorted, order, y, nullptr, HMOE_DT_BF16,
-                         stream);
+  rc = hmoe::down_scatter_at(act, wd, E, h, d, counts, HMOE_DT_I32, M, w_sorted, order, y, nullptr, HMOE_DT_BF16,
+                             stream, L.act_blocked);
   if (rc != HMOE_OK) return rc;
   return hmoe_combine(y, inv, T, k, d, out, HMOE_DT_BF16, stream);
 }
@@ -115,13 +121,14 @@ int hmoe_moe_forward(const void* x, int64_t ldx, const void* wr, const float* bi
 }  // extern "C"
 
 // The expert part for routing decided elsewhere (a model's own gate): hmoe_dispatch_tiles, hmoe_gate_up_swiglu(_tiles,
-// _i8) and hmoe_down_scatter(_i8) over one workspace, in the order and with the choices of the op-by-op path.
+// _i8) and hmoe_down_scatter(_i8) over one workspace, in the order and with the choices of the op-by-op path (but for the
+// layout of act, which no one else reads).
 namespace {
 
 struct ExpLayout {
   size_t counts, starts, order, a_idx, w_sorted, dws, tiles, act, total;
   size_t dws_bytes;
-  bool tiles_on;
+  bool tiles_on, act_blocked;
 };
 
 bool exp_layout(int64_t T, int64_t d, int E, int k, int64_t h, int w_dtype, int dtype, ExpLayout& L) {
@@ -144,7 +151,8 @@ bool exp_layout(int64_t T, int64_t d, int E, int k, int64_t h, int w_dtype, int 
   L.w_sorted = take(static_cast<size_t>(M) * 2);
   L.dws = take(L.dws_bytes);
   L.tiles = L.tiles_on ? take(tiles_bytes) : 0;
-  L.act = take(static_cast<size_t>(M) * static_cast<size_t>(h) * 2);
+  L.act_blocked = hmoe::act_blocked_rule(M, E, d, h, w_dtype == HMOE_DT_I8);
+  L.act = take(act_bytes(M, h, L.act_blocked));
   L.total = o;
   return true;
 }
@@ -194,17 +202,20 @@ int hmoe_moe_experts(const void* x, int64_t ldx, const void* topk_ids, int ids_d
                                stream);
   if (rc != HMOE_OK || M == 0) return rc;
   if (L.tiles_on)
-    rc = hmoe_gate_up_swiglu_tiles(tiles, wgu, E, d, h, counts, HMOE_DT_I32, M, act, nullptr, dtype, stream);
+    rc = hmoe::gate_up_swiglu_tiles_at(tiles, wgu, E, d, h, counts, HMOE_DT_I32, M, act, nullptr, dtype, stream,
+                                       L.act_blocked);
   else if (i8)
-    rc = hmoe_gate_up_swiglu_i8(x, ldx, a_idx, wgu, wgu_s, wgu_s_dtype, E, d, h, counts, HMOE_DT_I32, M, act, dtype,
-                                stream);
+    rc = hmoe::gate_up_swiglu_i8_at(x, ldx, a_idx, wgu, wgu_s, wgu_s_dtype, E, d, h, counts, HMOE_DT_I32, M, act,
+                                    dtype, stream, L.act_blocked);
   else
-    rc = hmoe_gate_up_swiglu(x, ldx, a_idx, wgu, E, d, h, counts, HMOE_DT_I32, M, act, nullptr, dtype, stream);
+    rc = hmoe::gate_up_swiglu_at(x, ldx, a_idx, wgu, E, d, h, counts, HMOE_DT_I32, M, act, nullptr, dtype, stream,
+                                 L.act_blocked);
   if (rc != HMOE_OK) return rc;
   if (i8)
-    return hmoe_down_scatter_i8(act, wd, wd_s, wd_s_dtype, E, h, d, counts, HMOE_DT_I32, M, w_sorted, order, y, dtype,
-                                stream);
-  return hmoe_down_scatter(act, wd, E, h, d, counts, HMOE_DT_I32, M, w_sorted, order, y, nullptr, dtype, stream);
+    return hmoe::down_scatter_i8_at(act, wd, wd_s, wd_s_dtype, E, h, d, counts, HMOE_DT_I32, M, w_sorted, order,
+                                    y, dtype, stream, L.act_blocked);
+  return hmoe::down_scatter_at(act, wd, E, h, d, counts, HMOE_DT_I32, M, w_sorted, order, y, nullptr, dtype, stream,
+                               L.act_blocked);
 }
 
 }  // extern "C"
