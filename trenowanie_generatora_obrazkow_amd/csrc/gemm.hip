@@ -1295,8 +1295,8 @@ bool act_blocked_rule(int64_t M, int64_t E, int64_t d, int64_t h, bool int8) {
          pick_few<EPI_STORE>(M, E, d, h, int8) == FEW_NONE;
 }
 
-int gate_up_swiglu_at(const void* x, int64_t ldx, const int32_t* a_idx, const void* wgu, int64_t E, int64_t d, int64_t
-                      h, const void* counts, int counts_dtype, int64_t M, void* act, void* gu, int dtype,
+int gate_up_swiglu_at(const void* x, int64_t ldx, const int32_t* a_idx, const void* wgu, int64_t E, int64_t d,
+                      int64_t h, const void* counts, int counts_dtype, int64_t M, void* act, void* gu, int dtype,
                       hmoe_stream_t stream, bool act_blocked) {
   int rc = check_common(counts, counts_dtype, E, M);
   if (rc) return rc;
@@ -1324,9 +1324,9 @@ int gate_up_swiglu_at(const void* x, int64_t ldx, const int32_t* a_idx, const vo
   return launch_fwd<EPI_SWIGLU>(p, h, f16, reinterpret_cast<hipStream_t>(stream));
 }
 
-int gate_up_swiglu_tiles_at(const void* xs_tiles, const void* wgu, int64_t E, int64_t d, int64_t h, const void*
-                            counts, int counts_dtype, int64_t M, void* act, void* gu, int dtype, hmoe_stream_t stream,
-                            bool act_blocked) {
+int gate_up_swiglu_tiles_at(const void* xs_tiles, const void* wgu, int64_t E, int64_t d, int64_t h,
+                            const void* counts, int counts_dtype, int64_t M, void* act, void* gu, int dtype,
+                            hmoe_stream_t stream, bool act_blocked) {
   int rc = check_common(counts, counts_dtype, E, M);
   if (rc) return rc;
   const bool f16 = act16(dtype, &rc);
@@ -1352,9 +1352,9 @@ int gate_up_swiglu_tiles_at(const void* xs_tiles, const void* wgu, int64_t E, in
   return launch_fwd<EPI_SWIGLU, true>(p, h, f16, reinterpret_cast<hipStream_t>(stream));
 }
 
-int down_scatter_at(const void* act, const void* wd, int64_t E, int64_t h, int64_t d, const void* counts, int
-                    counts_dtype, int64_t M, const uint16_t* w_sorted, const int32_t* y_idx, void* y, void* yhat, int
-                    dtype, hmoe_stream_t stream, bool act_blocked) {
+int down_scatter_at(const void* act, const void* wd, int64_t E, int64_t h, int64_t d, const void* counts,
+                    int counts_dtype, int64_t M, const uint16_t* w_sorted, const int32_t* y_idx, void* y, void* yhat,
+                    int dtype, hmoe_stream_t stream, bool act_blocked) {
   int rc = check_common(counts, counts_dtype, E, M);
   if (rc) return rc;
   const bool f16 = act16(dtype, &rc);
@@ -1383,9 +1383,9 @@ int down_scatter_at(const void* act, const void* wd, int64_t E, int64_t h, int64
   return act_blocked ? launch_fwd<EPI_STORE, true>(p, d, f16, s) : launch_fwd<EPI_STORE>(p, d, f16, s);
 }
 
-int gate_up_swiglu_i8_at(const void* x, int64_t ldx, const int32_t* a_idx, const void* wgu_q, const void* wgu_s, int
-                         wgu_s_dtype, int64_t E, int64_t d, int64_t h, const void* counts, int counts_dtype, int64_t
-                         M, void* act, int dtype, hmoe_stream_t stream, bool act_blocked) {
+int gate_up_swiglu_i8_at(const void* x, int64_t ldx, const int32_t* a_idx, const void* wgu_q, const void* wgu_s,
+                         int wgu_s_dtype, int64_t E, int64_t d, int64_t h, const void* counts, int counts_dtype,
+                         int64_t M, void* act, int dtype, hmoe_stream_t stream, bool act_blocked) {
   int rc = check_common(counts, counts_dtype, E, M);
   if (rc) return rc;
   const bool f16 = act16(dtype, &rc);
@@ -1416,8 +1416,8 @@ int gate_up_swiglu_i8_at(const void* x, int64_t ldx, const int32_t* a_idx, const
 }
 
 int down_scatter_i8_at(const void* act, const void* wd_q, const void* wd_s, int wd_s_dtype, int64_t E, int64_t h,
-                       int64_t d, const void* counts, int counts_dtype, int64_t M, const uint16_t* w_sorted, const
-                       int32_t* y_idx, void* y, int dtype, hmoe_stream_t stream, bool act_blocked) {
+                       int64_t d, const void* counts, int counts_dtype, int64_t M, const uint16_t* w_sorted,
+                       const int32_t* y_idx, void* y, int dtype, hmoe_stream_t stream, bool act_blocked) {
   int rc = check_common(counts, counts_dtype, E, M);
   if (rc) return rc;
   const bool f16 = act16(dtype, &rc);

@@ -29,21 +29,21 @@ inline int64_t blocked_bytes(int64_t M, int64_t h) { return tiles_bytes(M, 0, h)
 // act_blocked_rule: where both GEMMs are the persistent kernel's (the few-rows kernel keeps rows, which are few) and the
 // copies' 32-bit offsets reach.
 bool act_blocked_rule(int64_t M, int64_t E, int64_t d, int64_t h, bool int8);
-int gate_up_swiglu_at(const void* x, int64_t ldx, const int32_t* a_idx, const void* wgu, int64_t E, int64_t d, int64_t
-                      h, const void* counts, int counts_dtype, int64_t M, void* act, void* gu, int dtype,
+int gate_up_swiglu_at(const void* x, int64_t ldx, const int32_t* a_idx, const void* wgu, int64_t E, int64_t d,
+                      int64_t h, const void* counts, int counts_dtype, int64_t M, void* act, void* gu, int dtype,
                       hmoe_stream_t stream, bool act_blocked);
-int gate_up_swiglu_tiles_at(const void* xs_tiles, const void* wgu, int64_t E, int64_t d, int64_t h, const void*
-                            counts, int counts_dtype, int64_t M, void* act, void* gu, int dtype, hmoe_stream_t stream,
-                            bool act_blocked);
-int down_scatter_at(const void* act, const void* wd, int64_t E, int64_t h, int64_t d, const void* counts, int
-                    counts_dtype, int64_t M, const uint16_t* w_sorted, const int32_t* y_idx, void* y, void* yhat, int
-                    dtype, hmoe_stream_t stream, bool act_blocked);
-int gate_up_swiglu_i8_at(const void* x, int64_t ldx, const int32_t* a_idx, const void* wgu_q, const void* wgu_s, int
-                         wgu_s_dtype, int64_t E, int64_t d, int64_t h, const void* counts, int counts_dtype, int64_t
-                         M, void* act, int dtype, hmoe_stream_t stream, bool act_blocked);
+int gate_up_swiglu_tiles_at(const void* xs_tiles, const void* wgu, int64_t E, int64_t d, int64_t h,
+                            const void* counts, int counts_dtype, int64_t M, void* act, void* gu, int dtype,
+                            hmoe_stream_t stream, bool act_blocked);
+int down_scatter_at(const void* act, const void* wd, int64_t E, int64_t h, int64_t d, const void* counts,
+                    int counts_dtype, int64_t M, const uint16_t* w_sorted, const int32_t* y_idx, void* y, void* yhat,
+                    int dtype, hmoe_stream_t stream, bool act_blocked);
+int gate_up_swiglu_i8_at(const void* x, int64_t ldx, const int32_t* a_idx, const void* wgu_q, const void* wgu_s,
+                         int wgu_s_dtype, int64_t E, int64_t d, int64_t h, const void* counts, int counts_dtype,
+                         int64_t M, void* act, int dtype, hmoe_stream_t stream, bool act_blocked);
 int down_scatter_i8_at(const void* act, const void* wd_q, const void* wd_s, int wd_s_dtype, int64_t E, int64_t h,
-                       int64_t d, const void* counts, int counts_dtype, int64_t M, const uint16_t* w_sorted, const
-                       int32_t* y_idx, void* y, int dtype, hmoe_stream_t stream, bool act_blocked);
+                       int64_t d, const void* counts, int counts_dtype, int64_t M, const uint16_t* w_sorted,
+                       const int32_t* y_idx, void* y, int dtype, hmoe_stream_t stream, bool act_blocked);
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
