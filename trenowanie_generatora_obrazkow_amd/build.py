@@ -6,6 +6,11 @@ import subprocess
 import sys
 from concurrent.futures import ThreadPoolExecutor
 
+if __package__:
+    from . import isa_check
+else:  # run as a script
+    import isa_check
+
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB_DIR = os.path.join(HERE, "_lib")
@@ -50,6 +55,10 @@ def build(verbose: bool = False, extra_flags=()) -> str:
     if verbose:
         print(" ".join(cmd), flush=True)
     subprocess.run(cmd, check=True, capture_output=not verbose)
+    _, bad = isa_check.check(tmp)
+    if bad:
+        raise RuntimeError(f"{len(bad)} copies to LDS break a wait state rule (isa_check.py): "
+                           + "; ".join(f"{a:#x} {t}" for a, t in bad[:5]))
     os.replace(tmp, LIB)
     return LIB
 

@@ -103,7 +103,7 @@ __device__ __forceinline__ void buf2lds(uint32_t voff, i32x4 rsrc, uint32_t soff
 // matrix core for 32, so more than seven instructions between two MFMAs leave it idle, and a copy in buf2lds' form (the
 // generic pointer's null test, M0, five wait states) takes nine.  This form takes three: the scalar operands are used as
 // they are and only M0's own wait state is kept.  It relies on no VALU instruction writing one of its scalar operands in
-// the five wait states before it; the compiler cannot see that, so a test checks the built code for it.
+// the five wait states before it; the compiler cannot see that, so every build checks its code for it (isa_check.py).
 template <int OFF>
 __device__ __forceinline__ void buf2lds_inner(uint32_t voff, const i32x4& rsrc, uint32_t soff, uint32_t lds32) {
   asm volatile("s_add_u32 m0, %0, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
