@@ -268,6 +268,50 @@ def _rand_block(d, h, E, sh, seed):
     return m.to(torch.bfloat16)
 
 
+def test_poziomka_op_by_op_waits_on_its_own_streams(monkeypatch):
+    """The op-by-op block (with a probe set) beside a block call on another thread: whatever that thread records between
+    a record and a wait here, the side stream waits for this call's stream, and this call's stream for the side stream.
+    Streams and events are stand-ins that note which stream a wait watches."""
+    import contextlib
+
+    from trenowanie_generatora_obrazkow_amd import ops, poziomka
+    waits, shared_events = [], []
+
+    class Event:
+        def record(self, stream):
+            self.at = stream
+
+    class Stream:
+        def __init__(self, name):
+            self.name = name
+
+        def wait_event(self, ev):
+            for e in shared_events:  # the other thread's call comes in between
+                e.record(other)
+            waits.append((self.name, ev.at.name))
+
+        def wait_stream(self, stream):  # (an event made for this wait alone)
+            ev = Event()
+            ev.record(stream)
+            self.wait_event(ev)
+
+    main, side, other = Stream("main"), Stream("side"), Stream("other")
+    shared_events += [Event(), Event()]
+    monkeypatch.setattr(ops, "probe", {})
+    monkeypatch.setattr(ops, "side_stream", lambda dev: side)
+    monkeypatch.setattr(ops, "side_events", lambda dev: tuple(shared_events))
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda dev=None: main)
+    monkeypatch.setattr(torch.cuda, "stream", lambda s: contextlib.nullcontext())
+    monkeypatch.setattr(torch.Tensor, "record_stream", lambda self, s: None)
+    monkeypatch.setattr(poziomka, "_dense_swiglu", lambda x2, wgu, wd: waits.append("shared") or x2)
+    monkeypatch.setattr(ops, "route_sigmoid_group", lambda *a, **kw: (None, None, None))
+    monkeypatch.setattr(ops, "moe_experts", lambda *a, **kw: (None, None, None))
+    monkeypatch.setattr(ops, "combine", lambda y, T, k, add: waits.append("combine") or add)
+    m = _rand_block(64, 32, 8, 32, 0).to(torch.bfloat16)
+    m(torch.randn(4, 64).bfloat16())
+    assert waits == [("side", "main"), "shared", ("main", "side"), "combine"]
+
+
 def test_poziomka_export_round_trip(tmp_path):
     """load_export reads the layout export.py:62-102 writes (config.json lm_* fields; the fused trunk under "lm.",
     layer i's block under "lm.layers.{i}.mlp."), skips dense layers and other tensors, and export_state writes the same

@@ -25,12 +25,13 @@ def side_stream(device: torch.device):
     return _SIDE_STREAMS[key]
 
 
-_SIDE_EVENTS = {}  # device index -> (fork, join) events, reused by every fork to and join from the side stream
+_SIDE_EVENTS = {}  # device index -> (fork, join) events of every hmoe_moe_block call
 
 
 def side_events(device: torch.device):
-    """A (fork, join) pair of events per device for forking work onto the side stream and joining it back: recorded
-    and waited on in stream order, so one pair serves every fork (wait_stream would make a new event each time)."""
+    """A (fork, join) pair of events per device for forking work onto the side stream and joining it back: one pair
+    serves every fork of every thread (wait_stream would make a new event each time), so a record and the wait on it must
+    be one step under a lock, as hmoe_moe_block does it."""
     key = device.index if device.index is not None else torch.cuda.current_device()
     if key not in _SIDE_EVENTS:
         pair = (torch.cuda.Event(), torch.cuda.Event())

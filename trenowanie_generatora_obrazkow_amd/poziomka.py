@@ -164,13 +164,13 @@ class PoziomkaMoE(nn.Module):
             return ops.moe_block(x2, gw, gb, k, self.n_group, self.topk_group, self.scaling, self._wgu, self._wgu_s,
                                  self._wd, self._wd_s, wgu_sh, wd_sh, _one_count(T, x2.device),
                                  overlap=self.overlap_shared).view(shape)
-        # event timing of single ops (bench.py's probe) needs the launches apart: the same entry points one by one
+        # event timing of single ops (bench.py's probe) needs the launches apart: the same entry points one by one.  The
+        # fork and join make events of their own here: between a record of a shared event and the wait on it, a call of
+        # another thread may record it on its stream.
         side = ops.side_stream(x2.device) if self.overlap_shared and T > 0 else None
         if side is not None:  # fork: the shared expert needs only x
             main = torch.cuda.current_stream(x2.device)
-            fork_ev, join_ev = ops.side_events(x2.device)
-            fork_ev.record(main)
-            side.wait_event(fork_ev)
+            side.wait_stream(main)
             with torch.cuda.stream(side):
                 shared = _dense_swiglu(x2, wgu_sh, wd_sh)
             x2.record_stream(side)
@@ -179,8 +179,7 @@ class PoziomkaMoE(nn.Module):
         # dispatch, both int8 projections, routing weight and scatter in one C call
         y, _, _ = ops.moe_experts(x2, ids, w, self._wgu, self._wd, wgu_s=self._wgu_s, wd_s=self._wd_s)
         if side is not None:  # join before the combine reads the shared output
-            join_ev.record(side)
-            main.wait_event(join_ev)
+            main.wait_stream(side)
             shared.record_stream(main)
         else:
             shared = _dense_swiglu(x2, wgu_sh, wd_sh)
