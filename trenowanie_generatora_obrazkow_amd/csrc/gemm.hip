@@ -605,16 +605,15 @@ __global__ __launch_bounds__(C::NT, 1) void grouped_gemm_kernel(GemmParams p) {
         constexpr bool FAST = decltype(fast_tag)::value;
         // copies first .. first + n - 1 of slice ks, one per call of the returned function's gap
         auto copies = [&](auto first_tag, auto n_tag, int ks, bool on) {
-          constexpr int first = decltype(first_tag)::value, n = decltype(n_tag)::value;
           const int k0 = ks * kBK;
           const uint32_t sa = ta.soff_of(k0), sb = tb.soff_of(k0);
           const uint32_t pa = lds_addr(fill) + wave * (TA::PER_WAVE * 1024);
           const uint32_t pb = lds_addr(fill) + C::A_BYTES + wave * (TB::PER_WAVE * 1024);
           return [&, pa, pb, sa, sb, k0, on](int i) {
             if (!FAST && !on) return;
-            static_for<n>([&](auto lt) {
-              constexpr int l = first + decltype(lt)::value;
-              if (gap(decltype(lt)::value, n) != i) return;
+            static_for<decltype(n_tag)::value>([&](auto lt) {
+              constexpr int l = decltype(first_tag)::value + decltype(lt)::value;
+              if (gap(decltype(lt)::value, decltype(n_tag)::value) != i) return;
               if constexpr (!FAST)
                 copy_one(fill, l, k0);
               else if constexpr (l < TA::PER_WAVE)
