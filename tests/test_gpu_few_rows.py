@@ -67,3 +67,24 @@ def test_bit_identical_to_persistent(case, dt, quant, monkeypatch):
     want = run()
     for i, (a, b) in enumerate(zip(got, want)):
         assert torch.equal(a.view(torch.int16), b.view(torch.int16)), f"{case}: call {i}"
+
+
+@pytest.mark.parametrize("counts,M", [([70, 85, 15, 40], 90), ([3] * 100 + [90], 311), ([5, 40, 64, 64, 1, 2], 170)])
+def test_counts_beyond_the_rows(counts, M, monkeypatch):
+    """Counts that name more rows than there are: each expert's rows below M are its own, as in the persistent kernel."""
+    from trenowanie_generatora_obrazkow_amd import ops
+    print(f"few rows, counts of {sum(counts)} rows, M={M}", flush=True)
+    gen = torch.Generator().manual_seed(M)
+    E, K, N = len(counts), 96, 264
+    c = torch.tensor(counts, dtype=torch.int32).cuda()
+    x = torch.randn(M, K, generator=gen).bfloat16().cuda()
+    w = (torch.randn(E, K, N, generator=gen) * K ** -0.5).bfloat16().cuda()
+    got = ops.grouped_mm(x, w, c, M)
+    monkeypatch.setenv("HMOE_GEMM_TILE", "S")
+    assert torch.equal(got.view(torch.int16), ops.grouped_mm(x, w, c, M).view(torch.int16))
+    start = 0
+    for e, n in enumerate(counts):
+        r = slice(start, min(start + n, M))
+        start = min(start + n, M)
+        ref = x[r].float() @ w[e].float()
+        assert ((got[r].float() - ref).abs() <= 2 ** -8 * ref.abs() + 1e-4).all(), e

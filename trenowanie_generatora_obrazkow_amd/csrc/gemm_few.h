@@ -32,6 +32,7 @@ struct FewCfg {
 };
 constexpr int kFewMaxE = 256;           // experts: four per lane in the scan of the counts
 constexpr int64_t kFewMaxM = 1 << 20;  // rows (32-bit row arithmetic)
+static_assert(kFewMaxE * kFewMaxM < INT32_MAX, "sums of counts, each at most M");
 
 template <class C, int EPI, bool F16>
 __global__ __launch_bounds__(C::NT, 2) void few_rows_gemm_kernel(GemmParams p, int nb_n) {
@@ -62,7 +63,7 @@ __global__ __launch_bounds__(C::NT, 2) void few_rows_gemm_kernel(GemmParams p, i
     int64_t c = 0;
     if (i < per && e < E) c = read_count(p.counts, p.counts64, e);
     cnt[i] = (int)(c < 0 ? 0 : (c > p.M ? p.M : c));
-    rs = (int)min((int64_t)rs + cnt[i], p.M);  // (garbage counts must not overflow)
+    rs += cnt[i];  // (at most kFewMaxE * kFewMaxM, also where the counts name more rows than there are)
     ov += cnt[i] > 0 ? (cnt[i] - 1) / C::BM : 0;
   }
   int irs = rs, iov = ov;
@@ -70,7 +71,7 @@ __global__ __launch_bounds__(C::NT, 2) void few_rows_gemm_kernel(GemmParams p, i
   for (int s = 1; s < 64; s <<= 1) {
     const int a = __shfl_up(irs, s, 64), b = __shfl_up(iov, s, 64);
     if (lane >= s) {
-      irs = (int)min((int64_t)irs + a, p.M);
+      irs += a;
       iov += b;
     }
   }
