@@ -45,72 +45,69 @@ __global__ __launch_bounds__(C::NT, 2) void few_rows_gemm_kernel(GemmParams p, i
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int E = p.E;
 
-  // ---- the workgroup's tile: m-tiles [0, E) are the first one of their expert, the others the experts' further ones in
-  // order (at most M / BM of them).  Each wave scans the counts by itself, up to four experts per lane.
-  // Workgroups go to the 8 XCDs in turn: all n-tiles of an m-tile take ids of one XCD, next to each other, so that the
-  // weight lines two of them share (64-byte halves with int8 gate / up columns) are fetched into its L2 once.
-  const int q = (int)blockIdx.x >> 3;
-  int mt = (q / nb_n) * 8 + ((int)blockIdx.x & 7);
-  const int nb = q % nb_n;
-  const int Ep = (E + 7) & ~7;
-  if (mt >= E && mt < Ep) return;
-  if (mt >= Ep) mt -= Ep - E;
-  const int per = (E + 63) / 64;
-  int cnt[4], rs = 0, ov = 0;  // counts of the lane's experts; their rows, and their m-tiles after the first
+  // ---- the workgroup's tile.  The m-tiles, in expert order, are dealt to the 8 XCDs in runs (workgroups go to the XCDs in
+  // turn, so those with the same id modulo 8 share one), and all n-tiles of an m-tile follow each other: an expert's
+  // further m-tiles read its weights again soon after its first one and from the same L2, as do two n-tiles that share a
+  // weight line (64-byte halves with int8 gate / up columns).  Experts without rows take no tile, so the XCDs have equal
+  // shares whichever experts the tokens picked.  (Before, every expert's first m-tile came ahead of all further ones, expert
+  // e on XCD e % 8: up to 25% slower with the same tile where few experts have rows, a hot one has several tiles or the mean
+  // is 64 rows and more, within 2% elsewhere.)  Each wave scans the counts by itself, up to four experts per lane.
+  const int q = (int)blockIdx.x >> 3, nb = q % nb_n;
+  const int M = (int)p.M, per = (E + 63) / 64;
+  int cnt[4], rs = 0, tl = 0;  // counts of the lane's experts; their rows and m-tiles
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int e = lane * per + i;
     int64_t c = 0;
     if (i < per && e < E) c = read_count(p.counts, p.counts64, e);
-    cnt[i] = (int)(c < 0 ? 0 : (c > p.M ? p.M : c));
+    cnt[i] = (int)(c < 0 ? 0 : (c > M ? M : c));
     rs += cnt[i];  // (at most kFewMaxE * kFewMaxM, also where the counts name more rows than there are)
-    ov += cnt[i] > 0 ? (cnt[i] - 1) / C::BM : 0;
+    tl += (cnt[i] + C::BM - 1) / C::BM;
   }
-  int irs = rs, iov = ov;
+  int irs = rs, itl = tl;
 #pragma unroll
   for (int s = 1; s < 64; s <<= 1) {
-    const int a = __shfl_up(irs, s, 64), b = __shfl_up(iov, s, 64);
+    const int a = __shfl_up(irs, s, 64), b = __shfl_up(itl, s, 64);
     if (lane >= s) {
       irs += a;
-      iov += b;
+      itl += b;
     }
   }
-  int e, j = 0;  // expert and its m-tile
-  if (mt < E) {
-    e = mt;
-  } else {
-    const int want = mt - E;
-    const uint64_t owner = __ballot(iov > want);  // lanes are in expert order: the first one holds the tile
-    if (owner == 0) return;                       // (the same in both waves)
-    const int ol = __builtin_ctzll(owner);
-    int left = want - __shfl(iov - ov, ol, 64);
-    e = ol * per;
+  int st = irs - rs;  // the lane's first row
+  if (__builtin_amdgcn_readfirstlane(__shfl(irs, 63, 64)) > M) {  // more rows counted than there are: only those below M
+    tl = 0;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int c = __shfl(cnt[i], ol, 64);
-      const int t = c > 0 ? (c - 1) / C::BM : 0;
-      if (j == 0) {
-        if (left < t) {
-          j = left + 1;
-          e = ol * per + i;
-        } else {
-          left -= t;
-        }
-      }
+    for (int i = 0, r = st; i < 4; ++i) {
+      cnt[i] = max(0, min(cnt[i], M - r));
+      r += cnt[i];
+      tl += (cnt[i] + C::BM - 1) / C::BM;
+    }
+    itl = tl;
+#pragma unroll
+    for (int s = 1; s < 64; s <<= 1) {
+      const int b = __shfl_up(itl, s, 64);
+      if (lane >= s) itl += b;
     }
   }
-  int row0 = __shfl(irs - rs, e / per, 64), rows = 0;
+  const int total = __builtin_amdgcn_readfirstlane(__shfl(itl, 63, 64));
+  const int chunk = (total + 7) >> 3, at = q / nb_n, mt = ((int)blockIdx.x & 7) * chunk + at;
+  if (at >= chunk || mt >= total) return;
+  const int ol = __builtin_ctzll(__ballot(itl > mt));  // lanes are in expert order: the first one holds the tile
+  int left = mt - __shfl(itl - tl, ol, 64), first = __shfl(st, ol, 64), e = -1, row0 = 0, row_end = 0;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const int c = __shfl(cnt[i], e / per, 64);
-    if (i < e % per) row0 += c;
-    if (i == e % per) rows = c;
+    const int c = __shfl(cnt[i], ol, 64), t = (c + C::BM - 1) / C::BM;
+    if (e < 0 && left < t) {
+      e = ol * per + i;
+      row0 = first + left * C::BM;
+      row_end = min(first + c, row0 + C::BM);
+    }
+    left -= t;
+    first += c;
   }
-  row0 += j * C::BM;
   e = __builtin_amdgcn_readfirstlane(e);
   row0 = __builtin_amdgcn_readfirstlane(row0);
-  const int row_end = __builtin_amdgcn_readfirstlane((int)min((int64_t)row0 + min(rows - j * C::BM, C::BM), p.M));
-  if (row0 >= row_end) return;
+  row_end = __builtin_amdgcn_readfirstlane(row_end);
   const int n0 = nb * (EPI == EPI_SWIGLU ? C::BN / 2 : C::BN);
 
   // ---- copy sources ----
