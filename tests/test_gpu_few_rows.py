@@ -1,25 +1,27 @@
 """The few-rows GEMM kernel (csrc/gemm_few.h) against the persistent kernel, which the oracle tests pin: both run the same
 MFMAs in the same k order and round at the same places, so the results are equal bit for bit.  Sizes sit at the edges of
 its tiles (32, 64 and 128 rows; 128 and 256 columns), with empty experts, experts of several m-tiles, k-slices fewer than
-the ring holds, and ragged K and N."""
+the ring holds, ragged K and N, and row strides above the widths; the tile that the rule takes for them is checked."""
 import pytest
 import torch
 
 pytestmark = pytest.mark.gpu
 
-# rows per expert; (columns, K): chosen so that the rule takes the tile named (E, M and the columns decide)
-EDGE32 = [0, 1, 31, 32, 33, 0, 64, 5, 97]
+# rows per expert, columns, K, and the tile rows (0: the persistent kernel) that the rule takes for the products to N columns
+# with 16-bit and int8 weights, and for gate/up to N hidden columns with either
+EDGE32 = [0, 1, 31, 32, 33, 0, 64, 5, 97, 0, 0]
 CASES = {
-    "32x128-one-expert": ([40], 136, 72),
-    "32x128-edges": (EDGE32, 264, 1000),
-    "32x128-short-k": (EDGE32, 1024, 24),
-    "32x128-few-rows-many-experts": ([0] * 100 + [1, 0, 2] + [0] * 153, 512, 544),
-    "64x256-edges": ([0, 1, 63, 64, 65, 2, 0, 130] * 8, 520, 544),
-    "64x256-skew": ([600] + [3] * 60 + [0, 0, 0], 776, 40),
-    "64x256-256-experts": ([4, 0, 9, 7] * 64, 272, 96),
-    "128x256-edges": ([127, 128, 129, 0, 1, 64, 65, 200] * 4, 1304, 264),
-    "128x256-skew": ([1100] + [50] * 30 + [0], 1544, 64),
-    "257-experts": ([2, 1, 0] * 85 + [3, 1], 528, 136),  # past the kernel's expert limit: the persistent one
+    "one-expert": ([40], 136, 72, (32, 32, 32, 0)),
+    "32-row-edges": (EDGE32, 264, 744, (32, 32, 32, 32)),
+    "32-row-edges-short-k": (EDGE32, 1024, 24, (32, 32, 64, 64)),
+    "few-rows-many-experts": ([0] * 100 + [1, 0, 2] + [0] * 153, 512, 544, (32, 32, 32, 32)),
+    "64-row-edges": ([0, 1, 63, 64, 65, 2, 0, 130] * 8, 520, 544, (64, 64, 64, 64)),
+    "64-row-skew": ([600] + [3] * 60 + [0, 0, 0], 776, 40, (32, 64, 64, 64)),
+    "256-experts": ([4, 0, 9, 7] * 64, 272, 96, (32, 64, 64, 64)),
+    "128-row-edges": ([127, 128, 129, 0, 1, 64, 65, 200] * 4, 1928, 520, (128, 128, 128, 128)),
+    "128-row-skew": ([1100] + [50] * 30 + [0], 1976, 520, (128, 128, 128, 128)),
+    "128-row-short-k": ([1100] + [50] * 30 + [0], 1544, 64, (64, 64, 64, 128)),
+    "257-experts": ([2, 1, 0] * 85 + [3, 1], 528, 136, (0, 0, 0, 0)),  # past the kernel's expert limit
 }
 
 
@@ -45,25 +47,38 @@ def _weights(E, K, N, dt, quant, gen):
                                       (torch.float16, "fp32")])
 @pytest.mark.parametrize("case", CASES)
 def test_bit_identical_to_persistent(case, dt, quant, monkeypatch):
-    from trenowanie_generatora_obrazkow_amd import ops
-    counts, N, K = CASES[case]
+    from trenowanie_generatora_obrazkow_amd import _lib, ops
+    counts, N, K, tiles = CASES[case]
     N = -(-N // 16) * 16 if quant else N
+    tile = _lib.lib().hmoe_few_rows_tile
+    w_dt = _lib.dt(torch.int8 if quant else dt)
+    got = tile(sum(counts), len(counts), K, N, 0, w_dt), tile(sum(counts), len(counts), K, N, 1, w_dt)
+    assert got == (tiles[1::2] if quant else tiles[::2])
     print(f"few rows {case} {dt} quant={quant}", flush=True)
     gen = torch.Generator().manual_seed(len(case) + K)
     E, M, c, x, a_idx, y_idx, scale = _inputs(counts, dt, K, gen)
     w, ws = _weights(E, K, N, dt, quant, gen)
     wgu, gs = _weights(E, K, 2 * N, dt, quant, gen)
     xs = x[a_idx.long()].contiguous()
+    # the same operands with row strides above their widths
+    xw, ww = (torch.zeros(*t.shape[:-1], t.shape[-1] + 16, dtype=t.dtype, device="cuda") for t in (x, w))
+    xw[:, :K], ww[..., :N] = x, w
+    yw = torch.zeros(M, N + 24, dtype=dt, device="cuda")
 
     def run():
         return [ops.grouped_mm(x, w, c, M, a_idx=a_idx, y_idx=y_idx, scale=scale, w_scale=ws),
                 ops.grouped_mm(xs, w, c.long(), M, scale=scale.float(), w_scale=ws),
                 ops.down_scatter(xs, w, c, M, scale, y_idx, wd_s=ws)[0],
                 ops.gate_up_swiglu(x, wgu, c, M, a_idx=a_idx, wgu_s=gs)[0],
-                ops.gate_up_swiglu(xs, wgu, c, M, wgu_s=gs)[0]]
+                ops.gate_up_swiglu(xs, wgu, c, M, wgu_s=gs)[0],
+                ops.grouped_mm(xw[:, :K], ww[..., :N], c, M, a_idx=a_idx, y_idx=y_idx, scale=scale, w_scale=ws,
+                               out=yw[:, :N]).contiguous(),
+                ops.gate_up_swiglu(xw[:, :K], wgu, c, M, a_idx=a_idx, wgu_s=gs)[0]]
 
     got = run()
+    assert (yw[:, N:] == 0).all()
     monkeypatch.setenv("HMOE_GEMM_TILE", "S")
+    assert tile(M, E, K, N, 0, w_dt) == 0 and tile(M, E, K, N, 1, w_dt) == 0
     want = run()
     for i, (a, b) in enumerate(zip(got, want)):
         assert torch.equal(a.view(torch.int16), b.view(torch.int16)), f"{case}: call {i}"

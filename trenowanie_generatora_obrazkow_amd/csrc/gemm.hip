@@ -1162,34 +1162,59 @@ static int launch_few_tile(const GemmParams& p, int64_t ncols, hipStream_t s) {
   return HMOE_OK;
 }
 
-// The few-rows kernel (gemm_few.h) or the persistent one.  Measured on MI355X over 10 layers (d 256-2048, h 320-4096, 1-128
-// experts, bf16, fp16 and int8 weights), 2 to 768 routed rows per expert, gate/up and down, every tile against the
-// persistent kernel in one process, the weights of successive calls apart (read from HBM); us, persistent -> few:
-//   d 2048, h 320, 128 int8 experts: 8 rows per expert 61.8 -> 43.5 (gate/up) and 37.6 -> 27.6 (down), 48 rows 65.6 -> 55.4
-//   and 40 -> 34.4, 94 rows 78.8 -> 69.3 and 49.7 -> 49.8; d 2048, h 1408, 64 int8 experts: 2 rows 93 -> 67 and 50 -> 35,
-//   94 rows 121 -> 107 and 66 -> 57; d 1536, h 1024, 60 fp16 experts: 24 rows 75.9 -> 73 and 49 -> 44, 94 rows 87.8 -> 82.5
-//   and 57.2 -> 55.5; d 256, h 512, 8 experts: 94 rows 9.0 -> 6.9 and 10.0 -> 7.9.
-// Tiles: 64 rows x 256 columns up to 52 (16-bit weights: 40) rows per expert, above which experts often need a second tile,
-// which reads the weights again (48 rows, h 1408, int8 gate/up: 82 against 100 with 128-row tiles, whose copies of A cost
-// more beside half the weight bytes; 16-bit 76.0 / 76.2); then 128 x 256, or 64 x 256 where those leave too few workgroups.
-// 32 x 128 where they give no more than 3/4 of a workgroup per CU (1.5 with K up to 512: the launch is then a handful of
-// latencies long).  Above 112 (int8 gate/up: 132) rows per expert the products bound the launch and the persistent kernel's
-// 256-row tiles win (128 rows: fp16 gate/up 94 against 110, int8 down 64 / 68 and 75 / 84, int8 gate/up 89 / 77 and 148 /
-// 138; 160 rows: int8 gate/up 89 / 104 and 166 / 188).
-enum FewTile { FEW_NONE, FEW_32x128, FEW_64x256, FEW_128x256 };
+// The few-rows kernel (gemm_few.h) or the persistent one.  The rule sees the sizes, not the counts, so its lines lie where
+// the few-rows tile wins with even and with skewed counts alike: 270 layers drawn over d 256-2048, h 128-4160, 2-128 experts,
+// 1 to 200 rows per expert, even and Zipf 0.6-1.2 routing, every tile against the persistent kernel in one process, the
+// weights of successive calls apart (read from HBM).  Over these 13600 launches the tile taken is ahead by 8% (16-bit
+// gate/up), 12% (16-bit down), 19% and 25% (int8; geometric means), and more than 3% behind in 2.0, 0.7, 1.2 and 1.3% of
+// them; lines by the mean row count and an upper bound of the tiles had it behind in 12.5, 11.4, 5.2 and 3.9%, up to 1.7x.
+// us, persistent -> few, even counts (Zipf 1.2): d 2048, h 320, 128 int8 experts, 8 rows per expert 62.2 -> 43.5 (72.3 ->
+//   46.8) and 41.0 -> 27.1 (43.0 -> 27.3), 96 rows 80.4 -> 69.8 (98.6 -> 84.3) and 58.4 -> 54.9 (76.5 -> 54.6); d 2048, h 1408,
+//   64 int8 experts, 3 rows 91.2 -> 64.3 and 49.6 -> 35.1, 72 rows 116 -> 103 (137 -> 120) and 63.7 -> 53.5 (102 -> 83.4); d
+//   1536, h 1024, 60 16-bit experts, 9 rows down 47.5 -> 39.3 (48.9 -> 36.4), 51 rows 80.1 -> 76.0 (87.3 -> 88.0) and 51.9 ->
+//   46.8 (56.4 -> 51.8).
+// Workgroups per CU (by the experts that evenly routed rows hit) and the reduction's length decide.  A workgroup has two or
+// three slices in flight where the persistent kernel's has four, so below about one workgroup per CU a long reduction is
+// bound by their latency (4 experts, d 1600, 64 rows each, gate/up: 64x256 43 us, persistent 23), while a short one is over
+// before that counts.  16-bit weights need two or three per CU to gain anything over the persistent kernel, which streams
+// them at 4.8 TB/s; int8 weights, at half the bytes a slice, gain from 3/4 on.
+//   32 rows x 128 columns where there are few workgroups (each then has one m-tile and a share of the columns as small as
+//     possible), with 16-bit weights on gate/up only for a short reduction, or a row or two per expert where the persistent
+//     launch, which counts a tile per expert, would take large tiles; and up to 24 rows per expert on short reductions.
+//   64 x 256 up to 52 (int8: 44) rows per expert, above which experts often need a second m-tile; on a K up to 512 beyond it.
+//   128 x 256 from there to 112 rows per expert; above, the products bound the launch and the persistent kernel's 256-row
+//     tiles win.
+enum FewTile { FEW_NONE = 0, FEW_32x128 = 32, FEW_64x256 = 64, FEW_128x256 = 128 };
 template <int EPI>
 static FewTile pick_few(int64_t M, int64_t E, int64_t ncols, int64_t K, bool int8) {
-  if (E > kFewMaxE || M > kFewMaxM || env_force()) return FEW_NONE;
-  const int64_t cus = cu_count(), act = std::min(E, M);  // (at most M experts have rows)
+  constexpr bool GU = EPI == EPI_SWIGLU;
+  if (M <= 0 || E > kFewMaxE || M > kFewMaxM || env_force()) return FEW_NONE;
+  // (a grid's threads must stay below 2^32)
+  if ((E + M / 32 + 8) * ((ncols + 63) / 64) >= (1 << 23)) return FEW_NONE;
+  const int64_t cus = cu_count(), hit = std::min({E, M, E * M / (E + M) + 1});
   auto tiles = [&](int64_t bm, int64_t bn) {
-    const int64_t cols = EPI == EPI_SWIGLU ? bn / 2 : bn;
-    return (act + M / bm) * ((ncols + cols - 1) / cols);
+    const int64_t cols = GU ? bn / 2 : bn;
+    return (hit + M / bm) * ((ncols + cols - 1) / cols);
   };
-  const int64_t ta = tiles(32, 128);
-  if (ta * 4 <= cus * 3 || (ta * 2 <= cus * 3 && K <= 512)) return FEW_32x128;
-  if (M > E * (int8 && EPI == EPI_SWIGLU ? 132 : 112)) return FEW_NONE;
-  if (M > E * (int8 ? 52 : 40) && tiles(128, 256) >= cus) return FEW_128x256;
-  return tiles(64, 256) * 8 >= cus * 3 ? FEW_64x256 : FEW_NONE;
+  const int64_t t32 = tiles(32, 128), t64 = tiles(64, 256), t128 = tiles(128, 256);
+  auto rows_to = [&](int64_t per_expert) { return M <= E * per_expert; };
+  const bool thin = t32 * 4 <= cus * 3;  // at most 3/4 of a workgroup per CU
+  const bool large = pick_large_mgroup<EPI>(mgroup_tiles<CfgL, EPI>(M, E, ncols), ncols);
+  if (int8) {
+    const bool wide = t64 * 4 >= cus * (K > 512 ? 3 : 1) && rows_to(44);
+    if (GU ? !wide && large && t32 * 2 <= cus * 3 && rows_to(24) : t32 * 2 <= cus * 3 && (K <= 1024 || rows_to(24)))
+      return FEW_32x128;
+    if (GU && thin && K <= 1024 && rows_to(24)) return FEW_32x128;
+    if (wide) return FEW_64x256;
+    if (!rows_to(112)) return FEW_NONE;
+    if (!GU && K <= 512) return t64 * 4 >= cus ? FEW_64x256 : FEW_NONE;
+    return !rows_to(44) && t128 * 4 >= cus * 3 ? FEW_128x256 : FEW_NONE;
+  }
+  if (GU ? thin && (K <= 768 || (large && rows_to(2))) : thin || (K <= 1024 && rows_to(24))) return FEW_32x128;
+  if (!rows_to(112)) return FEW_NONE;
+  if (K <= 512) return (GU ? t32 <= cus : rows_to(40)) ? FEW_32x128 : FEW_64x256;
+  if (rows_to(52)) return t64 >= cus * (K > 1024 ? 3 : GU ? 2 : 1) ? FEW_64x256 : FEW_NONE;
+  return t128 * 2 >= cus * (K > 1024 ? 6 : 3) ? FEW_128x256 : FEW_NONE;
 }
 
 // launches the few-rows kernel if the rule picks it: *done, and the launch's status
@@ -1496,6 +1521,12 @@ int hmoe_grouped_mm(const void* a, int64_t lda, int a_dtype, const void* w, int 
     return launch_mgroup_i8<EPI_STORE>(p, N, f16, s);
   }
   return launch_fwd<EPI_STORE>(p, N, f16, s);
+}
+
+int hmoe_few_rows_tile(int64_t M, int64_t E, int64_t K, int64_t N, int swiglu, int w_dtype) {
+  if (M <= 0 || E <= 0 || K <= 0 || N <= 0) return 0;
+  const bool i8 = w_dtype == HMOE_DT_I8;
+  return swiglu ? pick_few<EPI_SWIGLU>(M, E, N, K, i8) : pick_few<EPI_STORE>(M, E, N, K, i8);
 }
 
 int hmoe_gate_up_swiglu(const void* x, int64_t ldx, const int32_t* a_idx, const void* wgu, int64_t E, int64_t d,
