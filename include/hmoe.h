@@ -162,10 +162,12 @@ int hmoe_grouped_mm(const void* a, int64_t lda, int a_dtype, const void* w, int 
                     const int32_t* a_idx, const int32_t* y_idx, const void* scale, int scale_dtype,
                     const void* w_scale, int w_scale_dtype, void* y, int64_t ldy, hmoe_stream_t stream);
 
-/* Rows of the tile that a forward grouped GEMM of these sizes runs on in the few-rows kernel (32, 64 or 128), or 0 where it
- * runs on the persistent kernel: swiglu 0 for hmoe_grouped_mm and hmoe_down_scatter(_i8) with N output columns, 1 for
- * hmoe_gate_up_swiglu(_i8) with N = h; K the reduction's length.  The results do not depend on it. */
-int hmoe_few_rows_tile(int64_t M, int64_t E, int64_t K, int64_t N, int swiglu, int w_dtype);
+/* The tile that a forward grouped GEMM of these sizes runs on: its rows (32, 64 or 128) in the few-rows kernel, minus its
+ * rows (-128 or -256) in the persistent kernel, 0 without work.  swiglu 0 for hmoe_grouped_mm and hmoe_down_scatter(_i8)
+ * with N output columns, 1 for hmoe_gate_up_swiglu(_i8) with N = h; K the reduction's length.  (A [g | u] or yhat output,
+ * row-group tiles of x, and act between the GEMMs of the one-call forms where neither runs on the few-rows kernel, take
+ * the persistent kernel.)  The results do not depend on it. */
+int hmoe_forward_tile(int64_t M, int64_t E, int64_t K, int64_t N, int swiglu, int w_dtype);
 
 /* Gate/up projection with the SwiGLU fused into the epilogue: replaces aurora/hf_compat.py:79 (grouped_mm(x,
  * _wgu, counts, sched, a_idx=a_idx).chunk(2)) and the self._act(g) * u of :81.

@@ -7,11 +7,11 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-# rows per expert, columns, K, and the tile rows (0: the persistent kernel) that the rule takes for the products to N columns
+# rows per expert, columns, K, and the tile rows (negative: the persistent kernel's) that the rule takes for the products to N columns
 # with 16-bit and int8 weights, and for gate/up to N hidden columns with either
 EDGE32 = [0, 1, 31, 32, 33, 0, 64, 5, 97, 0, 0]
 CASES = {
-    "one-expert": ([40], 136, 72, (32, 32, 32, 0)),
+    "one-expert": ([40], 136, 72, (32, 32, 32, -128)),
     "32-row-edges": (EDGE32, 264, 744, (32, 32, 32, 32)),
     "32-row-edges-short-k": (EDGE32, 1024, 24, (32, 32, 64, 64)),
     "few-rows-many-experts": ([0] * 100 + [1, 0, 2] + [0] * 153, 512, 544, (32, 32, 32, 32)),
@@ -21,7 +21,7 @@ CASES = {
     "128-row-edges": ([127, 128, 129, 0, 1, 64, 65, 200] * 4, 1928, 520, (128, 128, 128, 128)),
     "128-row-skew": ([1100] + [50] * 30 + [0], 1976, 520, (128, 128, 128, 128)),
     "128-row-short-k": ([1100] + [50] * 30 + [0], 1544, 64, (64, 64, 64, 128)),
-    "257-experts": ([2, 1, 0] * 85 + [3, 1], 528, 136, (0, 0, 0, 0)),  # past the kernel's expert limit
+    "257-experts": ([2, 1, 0] * 85 + [3, 1], 528, 136, (-128, -128, -256, -256)),  # past the kernel's expert limit
 }
 
 
@@ -50,7 +50,7 @@ def test_bit_identical_to_persistent(case, dt, quant, monkeypatch):
     from trenowanie_generatora_obrazkow_amd import _lib, ops
     counts, N, K, tiles = CASES[case]
     N = -(-N // 16) * 16 if quant else N
-    tile = _lib.lib().hmoe_few_rows_tile
+    tile = _lib.lib().hmoe_forward_tile
     w_dt = _lib.dt(torch.int8 if quant else dt)
     got = tile(sum(counts), len(counts), K, N, 0, w_dt), tile(sum(counts), len(counts), K, N, 1, w_dt)
     assert got == (tiles[1::2] if quant else tiles[::2])
@@ -78,7 +78,7 @@ def test_bit_identical_to_persistent(case, dt, quant, monkeypatch):
     got = run()
     assert (yw[:, N:] == 0).all()
     monkeypatch.setenv("HMOE_GEMM_TILE", "S")
-    assert tile(M, E, K, N, 0, w_dt) == 0 and tile(M, E, K, N, 1, w_dt) == 0
+    assert tile(M, E, K, N, 0, w_dt) == -128 and tile(M, E, K, N, 1, w_dt) == -128
     want = run()
     for i, (a, b) in enumerate(zip(got, want)):
         assert torch.equal(a.view(torch.int16), b.view(torch.int16)), f"{case}: call {i}"

@@ -37,7 +37,7 @@ SIGNATURES = {
     "hmoe_make_schedule": (_I32, [_P, _I32, _I32, _I64, _I32, _P, _P, _P, _P]),
     "hmoe_grouped_mm": (_I32, [_P, _I64, _I32, _P, _I32, _I64, _I64, _I64, _I64, _I64, _P, _I32, _I64, _P, _P, _P,
                                _I32, _P, _I32, _P, _I64, _P]),
-    "hmoe_few_rows_tile": (_I32, [_I64, _I64, _I64, _I64, _I32, _I32]),
+    "hmoe_forward_tile": (_I32, [_I64, _I64, _I64, _I64, _I32, _I32]),
     "hmoe_gate_up_swiglu": (_I32, [_P, _I64, _P, _P, _I64, _I64, _I64, _P, _I32, _I64, _P, _P, _I32, _P]),
     "hmoe_gate_up_swiglu_tiles": (_I32, [_P, _P, _I64, _I64, _I64, _P, _I32, _I64, _P, _P, _I32, _P]),
     "hmoe_xs_tiles_bytes": (_SZ, [_I64, _I32, _I64]),

@@ -1112,13 +1112,10 @@ static inline int64_t cu_count() {
 // spread over the CUs or pad much more of the output.
 //
 // Row-grouped launches: large tiles from 5/8 of a tile per CU on (160 tiles on 256 CUs): at 64-128 tiles small ones ran
-// 15-55% faster, from 160 tiles on large ones ran 10-57% faster, also at K = 320 (the h = 320 down GEMM, 20-47%).  int8
-// weights follow the same line since their conversions run in the MFMAs' shadow (large against small tiles, us: 128 experts,
-// h 320, 192 rows each gate/up 93 / 121 and down 75 / 86, 512 rows 210 / 258 and 198 / 198; 64 experts, h 1408, 192 rows
-// 174 / 244 and 89 / 120).  Once the large tiles give two per CU, small ones where the large would pad the output columns
-// by more than 10% (a SwiGLU n-tile with at most 64 live columns of 128 counts as 64: its main loop skips the dead half);
-// with fewer tiles the rounds they save matter more (the h = 320 down dgrad ran 53% faster on large tiles at 2048 tokens,
-// 3% slower at 8192).
+// 15-55% faster, from 160 tiles on large ones ran 10-57% faster, also at K = 320 (the h = 320 down GEMM, 20-47%).  Once the
+// large tiles give two per CU, small ones where the large would pad the output columns by more than 10% (a SwiGLU n-tile
+// with at most 64 live columns of 128 counts as 64: its main loop skips the dead half); with fewer tiles the rounds they save
+// matter more (the h = 320 down dgrad ran 53% faster on large tiles at 2048 tokens, 3% slower at 8192).
 template <int EPI>
 static bool pick_large_mgroup(int64_t tiles_large, int64_t ncols) {
   const int f = env_force();
@@ -1132,6 +1129,22 @@ static bool pick_large_mgroup(int64_t tiles_large, int64_t ncols) {
     if (padl * 10 > pads * 11) return false;
   }
   return tiles_large * 8 >= cus * 5;
+}
+
+// int8 weights (forward only): several small workgroups share a CU and hide each other's conversions, prologues and
+// epilogues, so on short reductions the small tiles stay ahead for longer; the large ones' conversions hide behind their own
+// MFMAs once there are enough of these.  Lines from 110 layers (d 256-2048, h 192-2560, 2-128 experts, even and Zipf 0.8
+// counts, from 80 rows per expert on), large against small in one process.  Large / small by tiles per CU (median):
+//   gate/up, K from 1024 on: 5/8 to 1 0.98-1.11, 1 to 1 1/2 0.80, 2 on 0.79; K 768-1023: 1 1/2 to 1 3/4 1.00, 1 3/4 on 0.87;
+//   K 512-767: 1 to 2 1/4 1.00, 2 1/4 on 0.92; K below 512: 1 to 3 1.00, 3 on 0.87.
+//   down, K from 512 on: 3/4 to 1 0.87, below up to 1.25; K below 512: 1 to 3 1.02-1.24, 3 to 6 1.02, 6 on 0.97.
+// By the 16-bit line 28% (gate/up) and 35% (down) of the launches with K below 512 and 12% of the other gate/up ones ran
+// more than 3% slower than with small tiles below 16 slices and, for gate/up, 2 1/2 tiles per CU; by these lines 2, 1 and 3%.
+template <int EPI>
+static bool pick_large_i8(int64_t tiles_large, int64_t ncols, int64_t K) {
+  if (const int f = env_force()) return f == 1;
+  const int eighths = EPI == EPI_SWIGLU ? (K >= 1024 ? 8 : K >= 768 ? 14 : K >= 512 ? 18 : 24) : (K >= 512 ? 5 : 48);
+  return pick_large_mgroup<EPI>(tiles_large, ncols) && tiles_large * 8 >= cu_count() * eighths;
 }
 
 template <int MODE, bool A_MN, bool B_MN, int EPI, bool A_BLK = false, bool F16 = false>
@@ -1180,7 +1193,7 @@ static int launch_few_tile(const GemmParams& p, int64_t ncols, hipStream_t s) {
 // them at 4.8 TB/s; int8 weights, at half the bytes a slice, gain from 3/4 on.
 //   32 rows x 128 columns where there are few workgroups (each then has one m-tile and a share of the columns as small as
 //     possible), with 16-bit weights on gate/up only for a short reduction, or a row or two per expert where the persistent
-//     launch, which counts a tile per expert, would take large tiles; and up to 24 rows per expert on short reductions.
+//     launch, which counts a tile per expert, could take large tiles; and up to 24 rows per expert on short reductions.
 //   64 x 256 up to 52 (int8: 44) rows per expert, above which experts often need a second m-tile; on a K up to 512 beyond it.
 //   128 x 256 from there to 112 rows per expert; above, the products bound the launch and the persistent kernel's 256-row
 //     tiles win.
@@ -1199,7 +1212,7 @@ static FewTile pick_few(int64_t M, int64_t E, int64_t ncols, int64_t K, bool int
   const int64_t t32 = tiles(32, 128), t64 = tiles(64, 256), t128 = tiles(128, 256);
   auto rows_to = [&](int64_t per_expert) { return M <= E * per_expert; };
   const bool thin = t32 * 4 <= cus * 3;  // at most 3/4 of a workgroup per CU
-  const bool large = pick_large_mgroup<EPI>(mgroup_tiles<CfgL, EPI>(M, E, ncols), ncols);
+  const bool large = mgroup_tiles<CfgL, EPI>(M, E, ncols) * 8 >= cus * 5;  // 5/8 of a large tile per CU by their bound
   if (int8) {
     const bool wide = t64 * 4 >= cus * (K > 512 ? 3 : 1) && rows_to(44);
     if (GU ? !wide && large && t32 * 2 <= cus * 3 && rows_to(24) : t32 * 2 <= cus * 3 && (K <= 1024 || rows_to(24)))
@@ -1252,7 +1265,7 @@ static int launch_mgroup_i8_t(const GemmParams& p, int64_t ncols, hipStream_t s)
     if (done) return rc;
   }
   const int64_t tl = mgroup_tiles<CfgL8, EPI>(p.M, p.E, ncols);
-  if (pick_large_mgroup<EPI>(tl, ncols)) return launch<CfgL8, MGROUP, false, true, EPI, A_BLK, F16>(p, tl, s);
+  if (pick_large_i8<EPI>(tl, ncols, p.K)) return launch<CfgL8, MGROUP, false, true, EPI, A_BLK, F16>(p, tl, s);
   return launch<CfgS8, MGROUP, false, true, EPI, A_BLK, F16>(p, mgroup_tiles<CfgS8, EPI>(p.M, p.E, ncols), s);
 }
 template <int EPI, bool A_BLK = false>
@@ -1523,10 +1536,16 @@ int hmoe_grouped_mm(const void* a, int64_t lda, int a_dtype, const void* w, int 
   return launch_fwd<EPI_STORE>(p, N, f16, s);
 }
 
-int hmoe_few_rows_tile(int64_t M, int64_t E, int64_t K, int64_t N, int swiglu, int w_dtype) {
+int hmoe_forward_tile(int64_t M, int64_t E, int64_t K, int64_t N, int swiglu, int w_dtype) {
   if (M <= 0 || E <= 0 || K <= 0 || N <= 0) return 0;
-  const bool i8 = w_dtype == HMOE_DT_I8;
-  return swiglu ? pick_few<EPI_SWIGLU>(M, E, N, K, i8) : pick_few<EPI_STORE>(M, E, N, K, i8);
+  auto rows = [&](auto epi_tag) -> int {
+    constexpr int EPI = decltype(epi_tag)::value;
+    const bool i8 = w_dtype == HMOE_DT_I8;
+    if (const FewTile few = pick_few<EPI>(M, E, N, K, i8)) return few;
+    const int64_t tl = mgroup_tiles<CfgL, EPI>(M, E, N);
+    return (i8 ? pick_large_i8<EPI>(tl, N, K) : pick_large_mgroup<EPI>(tl, N)) ? -CfgL::BM : -CfgS::BM;
+  };
+  return swiglu ? rows(std::integral_constant<int, EPI_SWIGLU>{}) : rows(std::integral_constant<int, EPI_STORE>{});
 }
 
 int hmoe_gate_up_swiglu(const void* x, int64_t ldx, const int32_t* a_idx, const void* wgu, int64_t E, int64_t d,
