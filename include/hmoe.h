@@ -307,9 +307,12 @@ int hmoe_down_dgrad_swiglu_dw(const void* dy, const int32_t* a_idx, const uint16
 int hmoe_gate_up_dgrad(const void* dgu, const void* wgu, int64_t E, int64_t d, int64_t h, const void* counts,
                        int counts_dtype, int64_t M, void* dxs, int dxs_dtype, hmoe_stream_t stream);
 
-/* The same with the reduction over 2h split into `parts` (fp32, each part's sum in its own (M, d) of dxs (parts, M, d)), for
- * row counts whose output has too few tiles to fill the chip; hmoe_unpermute_bwd_split adds the parts as it reads them.
- * hmoe_gate_up_dgrad_parts says how many parts these sizes are best split into (1: do not split). */
+/* The same with the reduction over 2h split into `parts` (fp32, each part's sum in its own (M, d) of dxs (parts, M, d), which
+ * so takes `parts` times the memory), for row counts whose output has too few tiles to fill the chip;
+ * hmoe_unpermute_bwd_split adds the parts as it reads them.  A part is a whole number of 32-wide k-slices, ceil(ceil(2h / 32)
+ * / parts) of them, the last one what is left; a count that leaves a part without a slice (2h = 288: 9 slices, 4 parts of
+ * 3) is refused with HMOE_ERR_ARG, as are parts < 1 and M * parts >= 2^31.  hmoe_gate_up_dgrad_parts says how many parts
+ * these sizes are best split into (1: do not split; at most 4, none of them empty). */
 int hmoe_gate_up_dgrad_parts(int64_t M, int64_t E, int64_t d, int64_t h);
 int hmoe_gate_up_dgrad_split(const void* dgu, const void* wgu, int64_t E, int64_t d, int64_t h, const void* counts,
                              int counts_dtype, int64_t M, float* dxs, int parts, hmoe_stream_t stream);

@@ -155,6 +155,50 @@ def test_argument_validation_codes(lib):
     assert L.hmoe_moe_experts_workspace_size(-1, 64, 8, 2, 64, BF, BF) == 0
 
 
+def test_split_dgrad_argument_codes(lib):
+    L = lib.lib()
+    P = 4096
+    split = lambda h, M, parts, dxs=P, dgu=P: L.hmoe_gate_up_dgrad_split(dgu, P, 3, 64, h, P, 4, M, dxs, parts, None)
+    assert split(144, 48, 0) == -1 and split(144, 48, -2) == -1
+    assert split(144, 48, 10) == -1  # more parts than the 9 slices of 2h = 288
+    assert split(144, 48, 4) == -1  # 4 parts of 3 slices: the last one is empty
+    assert split(144, (1 << 31) - 1, 2) == -1  # rows of all parts within 32 bits
+    assert split(144, 1 << 31, 2) == -2
+    assert split(144, 48, 2, dxs=None) == -1 and split(144, 48, 2, dxs=P + 8) == -1 and split(144, 48, 2, dgu=None) == -1
+    assert split(140, 48, 2) == -2  # h % 8
+    assert split(144, 0, 2) == 0  # no rows
+    # the parts that the query names are never refused
+    for M, E, d, h in ((4096, 8, 1024, 2048), (9003, 12, 760, 1352), (100, 4, 256, 264), (2000, 6, 512, 1032)):
+        parts = L.hmoe_gate_up_dgrad_parts(M, E, d, h)
+        slices = -(-2 * h // 32)
+        assert 1 <= parts <= 4 and -(-slices // -(-slices // parts)) == parts
+    assert L.hmoe_gate_up_dgrad_parts(0, 8, 1024, 2048) == 1
+    # un-permute of the parts
+    unp = lambda parts, d=64, dxs=P: L.hmoe_unpermute_bwd_split(dxs, parts, P, None, None, 4, 2, d, 0, P, None)
+    assert unp(0) == -1 and unp(2, d=60) == -1 and unp(2, dxs=None) == -1 and unp(2, dxs=P + 8) == -1
+    assert L.hmoe_unpermute_bwd_split(P, 2, P, None, None, 0, 2, 64, 0, P, None) == 0
+
+
+def test_block_call_argument_codes(lib):
+    L = lib.lib()
+    P, BF, I8 = 4096, 0, 5
+    size = lambda T=4, sh_h=32, k=2, w_dt=BF: L.hmoe_moe_block_workspace_size(T, 64, 8, k, 64, sh_h, w_dt)
+    ws = size()
+    assert ws > 0 and ws % 256 == 0 and size(T=0) == 0 and size(T=-1) == 0 and size(sh_h=0) == 0
+
+    def block(T=4, sh_h=32, sh_wgu=P, sh_wd=P, sh_count=P, out=P, x=P, ws_ptr=P, ws_b=ws, side=None, fork=None, join=None,
+              w_dt=BF, scales=None):
+        return L.hmoe_moe_block(x, 64, P, None, 4, 2, 2.5, P, scales, BF, P, scales, BF, w_dt, sh_wgu, sh_wd, sh_count,
+                                sh_h, T, 64, 8, 2, 64, out, ws_ptr, ws_b, None, side, fork, join)
+
+    assert block(T=0) == 0
+    assert block(T=-1) == -1 and block(sh_h=0) == -1
+    assert block(x=None) == -1 and block(out=None) == -1
+    assert block(sh_wgu=None) == -1 and block(sh_wd=None) == -1 and block(sh_count=None) == -1
+    assert block(side=P) == -1 and block(side=P, fork=P) == -1 and block(side=P, join=P) == -1  # a side stream, no events
+    assert block(ws_ptr=None) == -5 and block(ws_b=ws - 1) == -5 and block(ws_ptr=P + 64) == -5
+
+
 def test_workspace_queries(lib):
     L = lib.lib()
     a = L.hmoe_dispatch_workspace_size(16384, 2, 16)
