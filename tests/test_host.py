@@ -229,6 +229,36 @@ def test_moe_swiglu_rejects_mismatched_shapes_before_launch():
         moe_swiglu(x, wr, wgu, wd, 2, logit_bias=torch.zeros(E - 1))
 
 
+def test_moe_block_checks_the_shared_row_count(monkeypatch):
+    """ops.moe_block hands sh_count to a kernel that reads an int32 row count on the device: any other type, shape or
+    device stops on the host (the GPU checks and the call are stand-ins here)."""
+    from trenowanie_generatora_obrazkow_amd import ops
+    T, d, E, k, h, sh = 3, 32, 8, 2, 16, 16
+    bf = lambda *s: torch.zeros(*s, dtype=torch.bfloat16)
+    args = (bf(T, d), bf(E, d), torch.zeros(E), k, 4, 2, 2.5, bf(E, d, 2 * h), None, bf(E, h, d), None, bf(1, d, 2 * sh),
+            bf(1, sh, d))
+    calls, off_device = [], []
+
+    def require_gpu(t, name):
+        if any(t is o for o in off_device):
+            raise RuntimeError(f"{name} must be a ROCm GPU tensor")
+
+    monkeypatch.setattr(ops.L, "require_gpu", require_gpu)
+    monkeypatch.setattr(ops, "_dev_stream", lambda t: 0)
+    monkeypatch.setattr(ops.L, "call", lambda name, *a: calls.append(name))
+    count = torch.tensor([T], dtype=torch.int32)
+    ops.moe_block(*args, count, overlap=False)
+    assert calls == ["hmoe_moe_block"]
+    for bad, err in ((count.long(), TypeError), (torch.tensor([T, T], dtype=torch.int32), ValueError),
+                     (torch.tensor(T, dtype=torch.int32), ValueError), (None, ValueError)):
+        with pytest.raises(err):
+            ops.moe_block(*args, bad, overlap=False)
+    off_device.append(count)
+    with pytest.raises(RuntimeError, match="GPU"):
+        ops.moe_block(*args, count, overlap=False)
+    assert calls == ["hmoe_moe_block"]
+
+
 def test_poziomka_module_layout():
     """PoziomkaMoE keeps the reference's module tree, names, shapes and dtypes (aurora/hf_pipeline.py:314-346), so the
     reference's state dicts load unchanged; its forward refuses CPU tensors (no CPU path)."""
