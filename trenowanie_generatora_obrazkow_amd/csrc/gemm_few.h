@@ -3,12 +3,14 @@
 //
 // The persistent kernel (gemm.hip) gives a CU one 256x256 tile or two 128x128 ones: most of its ring and copy slots hold
 // rows of A, of which there are few here, and each tile's prologue (counts, expert scan, row ids), short main loop and
-// epilogue follow one another.  Here a workgroup is one tile of 32 FR rows x 64 columns per wave (SwiGLU: half of them gate
-// columns, half the matching up columns) and a CU holds two to six of them, so one fills its ring while another multiplies
-// or stores; what a tile's epilogue reads (row scatter index, routing weight, column scales) is loaded ahead of its first
-// copy.  Four waves side by side give 256-byte (16-bit) or 128-byte (int8) pieces of a gate row: half-line pieces measured
-// up to 25% slower.  A shallow ring and more workgroups per CU beat a deep ring (d 2048, h 320, 128 int8 experts, 4 rows
-// per expert, down: rings of 12, 8, 6, 5 and 4 slices with 32 rows 50.6, 36.4, 28.9, 23.8 and 22.7 us).
+// epilogue follow one another.  Here a workgroup is one tile of 32 FR rows x 64 columns per wave (two waves with 32 rows,
+// four otherwise; SwiGLU: half of the columns are gate columns, half the matching up ones) and a CU holds two to six of
+// them, so one fills its ring while another multiplies or stores; what a tile's epilogue reads (row scatter index, routing
+// weight, column scales) is loaded ahead of its first copy.  Four waves side by side give 256-byte (16-bit) or 128-byte
+// (int8) pieces of a gate row: half-line pieces measured up to 25% slower.  A shallow ring and more workgroups per CU beat a
+// deep ring (d 2048, h 320, 128 int8 experts, 4 rows per expert, down: rings of 12, 8, 6, 5 and 4 slices with 32 rows 50.6,
+// 36.4, 28.9, 23.8 and 22.7 us), but only with that many workgroups: with one per CU and a long reduction the two or three
+// slices in flight do not cover their latency, and the rule (gemm.hip) leaves such launches to the persistent kernel.
 // The ring is NS slices of 32 k deep with NS - 1 in flight; every iteration issues a whole slice (past K: copies outside
 // the range, which move nothing), so the wait counts are constants.
 //
@@ -135,7 +137,7 @@ __global__ __launch_bounds__(C::NT, 2) void few_rows_gemm_kernel(GemmParams p, i
     TB::slot(wave, lane, i, k, nn);
     int col = n0 + nn;
     bool ok = col < p.N;
-    if (EPI == EPI_SWIGLU) {  // tile columns [0, 64) gate, [64, 128) the matching up
+    if (EPI == EPI_SWIGLU) {  // tile columns [0, BN / 2) gate, [BN / 2, BN) the matching up
       const int ac = n0 + nn % (C::BN / 2);
       col = nn / (C::BN / 2) * p.h + ac;
       ok = ac < p.N;
@@ -145,7 +147,7 @@ __global__ __launch_bounds__(C::NT, 2) void few_rows_gemm_kernel(GemmParams p, i
   }
 
   // ---- epilogue inputs, loaded ahead of the copies: the lane's rows' scatter index and scale (row a*32 + lane%32), and
-  // with int8 weights its columns' scales (column halves b, groups g; a lane holds 4 consecutive columns per group) ----
+  // with int8 weights its columns' scales (halves b of BN / 2 columns, groups g; a lane holds 4 consecutive columns per group) ----
   [[maybe_unused]] int yr[C::FR];
   [[maybe_unused]] float sc[C::FR];
   if constexpr (EPI == EPI_STORE) {
@@ -261,7 +263,7 @@ __global__ __launch_bounds__(C::NT, 2) void few_rows_gemm_kernel(GemmParams p, i
   // bytes: with few rows the outputs are a few percent of the weights' bytes) ----
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
-    const int lc = wave * 32 + 8 * g + 4 * (lane >> 5);  // column within a 64-column half of the tile
+    const int lc = wave * 32 + 8 * g + 4 * (lane >> 5);  // column within a half (BN / 2) of the tile
     if constexpr (EPI == EPI_SWIGLU) {
       const int col = n0 + lc;
       if (col >= p.N) continue;

@@ -26,8 +26,10 @@ inline int64_t blocked_bytes(int64_t M, int64_t h) { return tiles_bytes(M, 0, h)
 // instruction (those cost the copy path about twice as much per byte).  Down GEMM, us, rows -> blocked:
 // 2048 tokens, d 1024, 8 experts, top-2, h 2048 (128x128 tiles) 50.7 -> 42.4; 8192 tokens, d 2048, 128 int8 experts, top-8,
 // h 320 197.7 -> 185.3; the gate/up launch stays within 3%.  (Not for training: the weight gradient reads act in rows.)
-// act_blocked_rule: where both GEMMs are the persistent kernel's (the few-rows kernel keeps rows, which are few) and the
-// copies' 32-bit offsets reach.
+// act_blocked_rule: where the few-rows rule leaves both GEMMs to the persistent kernel (the few-rows kernel reads and writes
+// rows, which are few) and the copies' 32-bit offsets reach.  It asks for a gate/up GEMM on x's own rows; one on row-group
+// tiles is the persistent kernel's in any case, and where only that GEMM's sizes would suit the few-rows kernel act stays
+// in rows.
 bool act_blocked_rule(int64_t M, int64_t E, int64_t d, int64_t h, bool int8);
 int gate_up_swiglu_at(const void* x, int64_t ldx, const int32_t* a_idx, const void* wgu, int64_t E, int64_t d,
                       int64_t h, const void* counts, int counts_dtype, int64_t M, void* act, void* gu, int dtype,
