@@ -1168,9 +1168,9 @@ static int launch_few_tile(const GemmParams& p, int64_t ncols, hipStream_t s) {
     attr_set[dev].store(true, std::memory_order_release);
   }
   const int64_t bn = EPI == EPI_SWIGLU ? C::BN / 2 : C::BN;
-  // an m-tile for every expert with rows and at most M / BM further ones, in eights (one per XCD)
-  const int64_t nb_n = (ncols + bn - 1) / bn, mt = (std::min<int64_t>(p.E, p.M) + p.M / C::BM + 7) / 8 * 8;
-  hipLaunchKernelGGL(kern, dim3((unsigned)(mt * nb_n)), dim3(C::NT), C::LDS_BYTES, s, p, (int)nb_n);
+  // an m-tile for every expert with rows and at most M / BM further ones; the tiles in eights (one per XCD)
+  const int64_t nb_n = (ncols + bn - 1) / bn, tiles = (std::min<int64_t>(p.E, p.M) + p.M / C::BM) * nb_n;
+  hipLaunchKernelGGL(kern, dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(C::NT), C::LDS_BYTES, s, p, (int)nb_n);
   HMOE_CHECK_LAUNCH();
   return HMOE_OK;
 }

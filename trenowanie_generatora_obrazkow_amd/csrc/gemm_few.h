@@ -47,14 +47,14 @@ __global__ __launch_bounds__(C::NT, 2) void few_rows_gemm_kernel(GemmParams p, i
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int E = p.E;
 
-  // ---- the workgroup's tile.  The m-tiles, in expert order, are dealt to the 8 XCDs in runs (workgroups go to the XCDs in
-  // turn, so those with the same id modulo 8 share one), and all n-tiles of an m-tile follow each other: an expert's
-  // further m-tiles read its weights again soon after its first one and from the same L2, as do two n-tiles that share a
-  // weight line (64-byte halves with int8 gate / up columns).  Experts without rows take no tile, so the XCDs have equal
-  // shares whichever experts the tokens picked.  (Before, every expert's first m-tile came ahead of all further ones, expert
-  // e on XCD e % 8: up to 25% slower with the same tile where few experts have rows, a hot one has several tiles or the mean
-  // is 64 rows and more, within 2% elsewhere.)  Each wave scans the counts by itself, up to four experts per lane.
-  const int q = (int)blockIdx.x >> 3, nb = q % nb_n;
+  // ---- the workgroup's tile.  The tiles, m-tiles in expert order and each with all its n-tiles in a row, are dealt to the 8
+  // XCDs in runs of equal length (workgroups go to the XCDs in turn, so those with the same id modulo 8 share one): the XCDs
+  // have equal shares whichever and however few experts the tokens picked, an expert's further m-tiles read its weights
+  // again soon after its first one and from the same L2, and so do two n-tiles that share a weight line (64-byte halves with
+  // int8 gate / up columns).  Same tile against whole m-tiles dealt to the XCDs in runs, 16-bit gate/up, geometric means:
+  // fewer than 8 rows per expert 0.92-0.97, 8 to 64 rows 0.95-0.99, 64 on 0.97 (one expert on one token, K 1024, h 4096: 19
+  // us, now 10); down projections within 1%.  (Every expert's first m-tile ahead of all further ones: 0.5-2.5% slower.)
+  // Each wave scans the counts by itself, up to four experts per lane.
   const int M = (int)p.M, per = (E + 63) / 64;
   int cnt[4], rs = 0, tl = 0;  // counts of the lane's experts; their rows and m-tiles
 #pragma unroll
@@ -92,8 +92,10 @@ __global__ __launch_bounds__(C::NT, 2) void few_rows_gemm_kernel(GemmParams p, i
     }
   }
   const int total = __builtin_amdgcn_readfirstlane(__shfl(itl, 63, 64));
-  const int chunk = (total + 7) >> 3, at = q / nb_n, mt = ((int)blockIdx.x & 7) * chunk + at;
-  if (at >= chunk || mt >= total) return;
+  const int share = (total * nb_n + 7) >> 3, at = (int)blockIdx.x >> 3;  // tiles per XCD, and the workgroup's in its run
+  const int tile = ((int)blockIdx.x & 7) * share + at;
+  if (at >= share || tile >= total * nb_n) return;
+  const int mt = tile / nb_n, nb = tile - mt * nb_n;
   const int ol = __builtin_ctzll(__ballot(itl > mt));  // lanes are in expert order: the first one holds the tile
   int left = mt - __shfl(itl - tl, ol, 64), first = __shfl(st, ol, 64), e = -1, row0 = 0, row_end = 0;
 #pragma unroll
