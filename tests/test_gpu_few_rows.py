@@ -11,16 +11,16 @@ pytestmark = pytest.mark.gpu
 # with 16-bit and int8 weights, and for gate/up to N hidden columns with either
 EDGE32 = [0, 1, 31, 32, 33, 0, 64, 5, 97, 0, 0]
 CASES = {
-    "one-expert": ([40], 136, 72, (32, 32, 32, -128)),
+    "one-expert": ([40], 136, 72, (32, 32, 32, 32)),
     "32-row-edges": (EDGE32, 264, 744, (32, 32, 32, 32)),
-    "32-row-edges-short-k": (EDGE32, 1024, 24, (32, 32, 64, 64)),
+    "32-row-edges-short-k": (EDGE32, 1024, 24, (32, 32, 32, 32)),
     "few-rows-many-experts": ([0] * 100 + [1, 0, 2] + [0] * 153, 512, 544, (32, 32, 32, 32)),
     "64-row-edges": ([0, 1, 63, 64, 65, 2, 0, 130] * 8, 520, 544, (64, 64, 64, 64)),
-    "64-row-skew": ([600] + [3] * 60 + [0, 0, 0], 776, 40, (32, 64, 64, 64)),
-    "256-experts": ([4, 0, 9, 7] * 64, 272, 96, (32, 64, 64, 64)),
+    "64-row-skew": ([600] + [3] * 60 + [0, 0, 0], 1976, 40, (64, 64, 64, 64)),
+    "256-experts": ([4, 0, 9, 7] * 64, 272, 96, (32, 32, 64, 64)),
     "128-row-edges": ([127, 128, 129, 0, 1, 64, 65, 200] * 4, 1928, 520, (128, 128, 128, 128)),
     "128-row-skew": ([1100] + [50] * 30 + [0], 1976, 520, (128, 128, 128, 128)),
-    "128-row-short-k": ([1100] + [50] * 30 + [0], 1544, 64, (64, 64, 64, 128)),
+    "128-row-short-k": ([1100] + [50] * 30 + [0], 1544, 64, (64, 64, 128, 128)),
     "257-experts": ([2, 1, 0] * 85 + [3, 1], 528, 136, (-128, -128, -256, -256)),  # past the kernel's expert limit
 }
 

@@ -508,13 +508,12 @@ def test_forward_tile_rule():
     from trenowanie_generatora_obrazkow_amd import _lib
     BF, I8 = _lib.dt(torch.bfloat16), _lib.dt(torch.int8)
     tile = _lib.lib().hmoe_forward_tile  # (M, E, K, N, swiglu, weight type)
-    # less than about a workgroup per CU on a long reduction: the persistent kernel
-    assert tile(256, 4, 1600, 3200, 1, BF) < 0 and tile(64, 1, 1024, 4096, 1, BF) < 0
-    assert tile(512, 17, 1840, 1552, 1, BF) < 0 and tile(768, 9, 1320, 3216, 1, BF) < 0
-    # 16-bit weights, one or two workgroups per CU: the persistent kernel
-    assert tile(4096, 42, 1360, 1504, 0, BF) < 0 and tile(16, 19, 1536, 2720, 1, BF) < 0
+    # more workgroups than the persistent kernel's rounds have use for, or few on small tiles: the persistent kernel
+    assert tile(1536, 21, 3632, 920, 0, BF) < 0 and tile(4096, 25, 2048, 4096, 1, BF) < 0
     # many products per weight: the persistent kernel
     assert tile(128 * 113, 128, 2048, 320, 1, I8) < 0 and tile(60 * 113, 60, 1536, 1024, 1, BF) < 0
+    # few tokens over few wide experts
+    assert tile(16, 4, 1600, 3200, 1, BF) == 32 and tile(4, 1, 1024, 4096, 1, BF) == 32
     # int8 experts on prompts and on a batch of captions
     assert tile(512, 128, 2048, 320, 1, I8) == 64 and tile(512, 128, 320, 2048, 0, I8) == 64
     assert tile(12000, 128, 2048, 320, 1, I8) == 128 and tile(144, 64, 2048, 1408, 1, I8) == 64
@@ -527,5 +526,5 @@ def test_forward_tile_rule():
     assert tile(0, 8, 512, 1024, 0, BF) == 0
     # int8 on large tiles of the persistent kernel: by the reduction's length and tiles per CU
     assert tile(128 * 192, 128, 2048, 320, 1, I8) == -256 and tile(128 * 512, 128, 320, 2048, 0, I8) == -256
-    assert tile(26 * 132, 26, 528, 960, 1, I8) == -128 and tile(16 * 207, 16, 768, 256, 1, I8) == -128
-    assert tile(36 * 128, 36, 352, 1568, 0, I8) == -128 and tile(23 * 384, 23, 224, 1632, 0, I8) == -128
+    assert tile(26 * 140, 26, 528, 960, 1, I8) == -128 and tile(16 * 207, 16, 512, 256, 1, I8) == -128
+    assert tile(36 * 140, 36, 352, 1568, 0, I8) == -128 and tile(23 * 384, 23, 224, 1632, 0, I8) == -128

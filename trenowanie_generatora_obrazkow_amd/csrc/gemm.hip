@@ -1135,15 +1135,15 @@ static bool pick_large_mgroup(int64_t tiles_large, int64_t ncols) {
 // epilogues, so on short reductions the small tiles stay ahead for longer; the large ones' conversions hide behind their own
 // MFMAs once there are enough of these.  Lines from 110 layers (d 256-2048, h 192-2560, 2-128 experts, even and Zipf 0.8
 // counts, from 80 rows per expert on), large against small in one process.  Large / small by tiles per CU (median):
-//   gate/up, K from 1024 on: 5/8 to 1 0.98-1.11, 1 to 1 1/2 0.80, 2 on 0.79; K 768-1023: 1 1/2 to 1 3/4 1.00, 1 3/4 on 0.87;
-//   K 512-767: 1 to 2 1/4 1.00, 2 1/4 on 0.92; K below 512: 1 to 3 1.00, 3 on 0.87.
-//   down, K from 512 on: 3/4 to 1 0.87, below up to 1.25; K below 512: 1 to 3 1.02-1.24, 3 to 6 1.02, 6 on 0.97.
+//   gate/up, K from 768 on: 5/8 to 3/4 1.1, 3/4 to 1 0.87-0.98, 1 to 1 1/2 0.78-0.89, 2 on 0.79-0.89; K 512-767: 1 to 2 1/4
+//     1.00, 2 1/4 on 0.92; K 384-511: 1 1/2 to 2 1/4 0.97-1.04, 2 1/4 on 0.88; K below 384: 1 to 3 1.04, 3 on 0.93.
+//   down, K from 512 on: 5/8 to 3/4 1.14-1.37, 3/4 on 0.87-1.1; K below 512: 1 to 3 1.02-1.24, 3 to 6 1.02, 6 on 0.97.
 // By the 16-bit line 28% (gate/up) and 35% (down) of the launches with K below 512 and 12% of the other gate/up ones ran
-// more than 3% slower than with small tiles below 16 slices and, for gate/up, 2 1/2 tiles per CU; by these lines 2, 1 and 3%.
+// more than 3% slower than with small tiles below 16 slices and, for gate/up, 2 1/2 tiles per CU; by these lines 2, 1 and 5%.
 template <int EPI>
 static bool pick_large_i8(int64_t tiles_large, int64_t ncols, int64_t K) {
   if (const int f = env_force()) return f == 1;
-  const int eighths = EPI == EPI_SWIGLU ? (K >= 1024 ? 8 : K >= 768 ? 14 : K >= 512 ? 18 : 24) : (K >= 512 ? 5 : 48);
+  const int eighths = EPI == EPI_SWIGLU ? (K >= 768 ? 7 : K >= 384 ? 18 : 24) : (K >= 512 ? 6 : 48);
   return pick_large_mgroup<EPI>(tiles_large, ncols) && tiles_large * 8 >= cu_count() * eighths;
 }
 
@@ -1178,25 +1178,19 @@ static int launch_few_tile(const GemmParams& p, int64_t ncols, hipStream_t s) {
 // The few-rows kernel (gemm_few.h) or the persistent one.  The rule sees the sizes, not the counts, so its lines lie where
 // the few-rows tile wins with even and with skewed counts alike: 270 layers drawn over d 256-2048, h 128-4160, 2-128 experts,
 // 1 to 200 rows per expert, even and Zipf 0.6-1.2 routing, every tile against the persistent kernel in one process, the
-// weights of successive calls apart (read from HBM).  Over these 13600 launches the tile taken is ahead by 8% (16-bit
-// gate/up), 12% (16-bit down), 19% and 25% (int8; geometric means), and more than 3% behind in 2.0, 0.7, 1.2 and 1.3% of
-// them; lines by the mean row count and an upper bound of the tiles had it behind in 12.5, 11.4, 5.2 and 3.9%, up to 1.7x.
-// us, persistent -> few, even counts (Zipf 1.2): d 2048, h 320, 128 int8 experts, 8 rows per expert 62.2 -> 43.5 (72.3 ->
-//   46.8) and 41.0 -> 27.1 (43.0 -> 27.3), 96 rows 80.4 -> 69.8 (98.6 -> 84.3) and 58.4 -> 54.9 (76.5 -> 54.6); d 2048, h 1408,
-//   64 int8 experts, 3 rows 91.2 -> 64.3 and 49.6 -> 35.1, 72 rows 116 -> 103 (137 -> 120) and 63.7 -> 53.5 (102 -> 83.4); d
-//   1536, h 1024, 60 16-bit experts, 9 rows down 47.5 -> 39.3 (48.9 -> 36.4), 51 rows 80.1 -> 76.0 (87.3 -> 88.0) and 51.9 ->
-//   46.8 (56.4 -> 51.8).
-// Workgroups per CU (by the experts that evenly routed rows hit) and the reduction's length decide.  A workgroup has two or
-// three slices in flight where the persistent kernel's has four, so below about one workgroup per CU a long reduction is
-// bound by their latency (4 experts, d 1600, 64 rows each, gate/up: 64x256 43 us, persistent 23), while a short one is over
-// before that counts.  16-bit weights need two or three per CU to gain anything over the persistent kernel, which streams
-// them at 4.8 TB/s; int8 weights, at half the bytes a slice, gain from 3/4 on.
-//   32 rows x 128 columns where there are few workgroups (each then has one m-tile and a share of the columns as small as
-//     possible), with 16-bit weights on gate/up only for a short reduction, or a row or two per expert where the persistent
-//     launch, which counts a tile per expert, could take large tiles; and up to 24 rows per expert on short reductions.
-//   64 x 256 up to 52 (int8: 44) rows per expert, above which experts often need a second m-tile; on a K up to 512 beyond it.
-//   128 x 256 from there to 112 rows per expert; above, the products bound the launch and the persistent kernel's 256-row
-//     tiles win.
+// weights of successive calls apart (read from HBM).  Over these 13600 launches the choice takes 0.84 (16-bit gate/up), 0.85
+// (16-bit down), 0.80 and 0.79 (int8) of the persistent kernel's time in the geometric mean (the best tile of each launch:
+// 0.80, 0.82, 0.77, 0.77), and more than 3% longer in 1.9, 1.3, 1.0 and 3.4% of them; lines by the mean row count alone, 0.85,
+// 0.90, 0.80 and 0.81, in 5.8, 11.1, 5.2 and 6.7%.
+// What decides is how many workgroups a CU gets, with one m-tile for each expert that evenly routed rows would hit:
+//   32 rows x 128 columns up to 5/4 of them per CU (the launch is then one chain of latencies, and small tiles share it out
+//     over most CUs), and up to 3 on down projections of short reductions with up to 24 rows per expert;
+//   64 x 256 and 128 x 256 up to 7/5 of them per CU for every round of the persistent kernel (its large tiles come one to a
+//     CU, its small ones two): from there on the rounds' full tiles are the better use of the CUs.  Below 3/4 per CU 64 x
+//     256 only where that kernel would take large tiles.  With K up to 512 64 x 256 in any case: prologue and epilogue, which
+//     the few-rows workgroups of a CU hide from each other, are then most of a tile's time;
+//   128 x 256 above 52 rows per expert, where experts often need a second m-tile, which reads the weights again, with at
+//     least one per CU; none above 112, where the products bound the launch and 256-row tiles win.
 enum FewTile { FEW_NONE = 0, FEW_32x128 = 32, FEW_64x256 = 64, FEW_128x256 = 128 };
 template <int EPI>
 static FewTile pick_few(int64_t M, int64_t E, int64_t ncols, int64_t K, bool int8) {
@@ -1210,24 +1204,14 @@ static FewTile pick_few(int64_t M, int64_t E, int64_t ncols, int64_t K, bool int
     return (hit + M / bm) * ((ncols + cols - 1) / cols);
   };
   const int64_t t32 = tiles(32, 128), t64 = tiles(64, 256), t128 = tiles(128, 256);
+  const int64_t tl = mgroup_tiles<CfgL, EPI>(M, E, ncols);
+  const bool large = int8 ? pick_large_i8<EPI>(tl, ncols, K) : pick_large_mgroup<EPI>(tl, ncols);
+  const int64_t rounds = large ? (tiles(256, 256) + cus - 1) / cus : (tiles(128, 128) + 2 * cus - 1) / (2 * cus);
   auto rows_to = [&](int64_t per_expert) { return M <= E * per_expert; };
-  const bool thin = t32 * 4 <= cus * 3;  // at most 3/4 of a workgroup per CU
-  const bool large = mgroup_tiles<CfgL, EPI>(M, E, ncols) * 8 >= cus * 5;  // 5/8 of a large tile per CU by their bound
-  if (int8) {
-    const bool wide = t64 * 4 >= cus * (K > 512 ? 3 : 1) && rows_to(44);
-    if (GU ? !wide && large && t32 * 2 <= cus * 3 && rows_to(24) : t32 * 2 <= cus * 3 && (K <= 1024 || rows_to(24)))
-      return FEW_32x128;
-    if (GU && thin && K <= 1024 && rows_to(24)) return FEW_32x128;
-    if (wide) return FEW_64x256;
-    if (!rows_to(112)) return FEW_NONE;
-    if (!GU && K <= 512) return t64 * 4 >= cus ? FEW_64x256 : FEW_NONE;
-    return !rows_to(44) && t128 * 4 >= cus * 3 ? FEW_128x256 : FEW_NONE;
-  }
-  if (GU ? thin && (K <= 768 || (large && rows_to(2))) : thin || (K <= 1024 && rows_to(24))) return FEW_32x128;
+  if (t32 * 4 <= cus * 5 || (!GU && K <= 1280 && rows_to(24) && t32 <= 3 * cus)) return FEW_32x128;
   if (!rows_to(112)) return FEW_NONE;
-  if (K <= 512) return (GU ? t32 <= cus : rows_to(40)) ? FEW_32x128 : FEW_64x256;
-  if (rows_to(52)) return t64 >= cus * (K > 1024 ? 3 : GU ? 2 : 1) ? FEW_64x256 : FEW_NONE;
-  return t128 * 2 >= cus * (K > 1024 ? 6 : 3) ? FEW_128x256 : FEW_NONE;
+  if (!rows_to(52) && (GU || K > 512) && t128 >= cus && t128 * 5 <= 7 * cus * rounds) return FEW_128x256;
+  return K <= 512 || ((large || t64 * 4 >= 3 * cus) && t64 * 5 <= 7 * cus * rounds) ? FEW_64x256 : FEW_NONE;
 }
 
 // launches the few-rows kernel if the rule picks it: *done, and the launch's status
