@@ -511,7 +511,7 @@ def test_forward_tile_rule():
     # more workgroups than the persistent kernel's rounds have use for, or few on small tiles: the persistent kernel
     assert tile(1536, 21, 3632, 920, 0, BF) < 0 and tile(4096, 25, 2048, 4096, 1, BF) < 0
     # many products per weight: the persistent kernel
-    assert tile(128 * 113, 128, 2048, 320, 1, I8) < 0 and tile(60 * 113, 60, 1536, 1024, 1, BF) < 0
+    assert tile(128 * 133, 128, 2048, 320, 1, I8) < 0 and tile(60 * 113, 60, 1536, 1024, 1, BF) < 0
     # few tokens over few wide experts
     assert tile(16, 4, 1600, 3200, 1, BF) == 32 and tile(4, 1, 1024, 4096, 1, BF) == 32
     # int8 experts on prompts and on a batch of captions

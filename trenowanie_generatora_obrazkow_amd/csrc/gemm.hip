@@ -1189,8 +1189,9 @@ static int launch_few_tile(const GemmParams& p, int64_t ncols, hipStream_t s) {
 //     CU, its small ones two): from there on the rounds' full tiles are the better use of the CUs.  Below 3/4 per CU 64 x
 //     256 only where that kernel would take large tiles.  With K up to 512 64 x 256 in any case: prologue and epilogue, which
 //     the few-rows workgroups of a CU hide from each other, are then most of a tile's time;
-//   128 x 256 above 52 rows per expert, where experts often need a second m-tile, which reads the weights again, with at
-//     least one per CU; none above 112, where the products bound the launch and 256-row tiles win.
+//   128 x 256 above 52 rows per expert, where experts often need a second m-tile, which reads the weights again, or where 64 x
+//     256 are too many, with at least one per CU; none above 112 (int8 gate/up 132), where the products bound the launch
+//     and 256-row tiles win.
 enum FewTile { FEW_NONE = 0, FEW_32x128 = 32, FEW_64x256 = 64, FEW_128x256 = 128 };
 template <int EPI>
 static FewTile pick_few(int64_t M, int64_t E, int64_t ncols, int64_t K, bool int8) {
@@ -1203,15 +1204,17 @@ static FewTile pick_few(int64_t M, int64_t E, int64_t ncols, int64_t K, bool int
     const int64_t cols = GU ? bn / 2 : bn;
     return (hit + M / bm) * ((ncols + cols - 1) / cols);
   };
-  const int64_t t32 = tiles(32, 128), t64 = tiles(64, 256), t128 = tiles(128, 256);
+  auto rows_to = [&](int64_t per_expert) { return M <= E * per_expert; };
+  const int64_t t32 = tiles(32, 128);
+  if (t32 * 4 <= cus * 5 || (!GU && K <= 1280 && rows_to(24) && t32 <= 3 * cus)) return FEW_32x128;
+  if (!rows_to(int8 && GU ? 132 : 112)) return FEW_NONE;
   const int64_t tl = mgroup_tiles<CfgL, EPI>(M, E, ncols);
   const bool large = int8 ? pick_large_i8<EPI>(tl, ncols, K) : pick_large_mgroup<EPI>(tl, ncols);
   const int64_t rounds = large ? (tiles(256, 256) + cus - 1) / cus : (tiles(128, 128) + 2 * cus - 1) / (2 * cus);
-  auto rows_to = [&](int64_t per_expert) { return M <= E * per_expert; };
-  if (t32 * 4 <= cus * 5 || (!GU && K <= 1280 && rows_to(24) && t32 <= 3 * cus)) return FEW_32x128;
-  if (!rows_to(112)) return FEW_NONE;
-  if (!rows_to(52) && (GU || K > 512) && t128 >= cus && t128 * 5 <= 7 * cus * rounds) return FEW_128x256;
-  return K <= 512 || ((large || t64 * 4 >= 3 * cus) && t64 * 5 <= 7 * cus * rounds) ? FEW_64x256 : FEW_NONE;
+  const int64_t t64 = tiles(64, 256), t128 = tiles(128, 256), most = 7 * cus * rounds;  // (fifths)
+  const bool fit64 = (large || t64 * 4 >= 3 * cus) && t64 * 5 <= most, fit128 = t128 >= cus && t128 * 5 <= most;
+  if ((GU || K > 512) && fit128 && !(fit64 && rows_to(52))) return FEW_128x256;
+  return fit64 || K <= 512 ? FEW_64x256 : FEW_NONE;
 }
 
 // launches the few-rows kernel if the rule picks it: *done, and the launch's status
