@@ -1117,10 +1117,7 @@ static inline int64_t cu_count() {
 // with at most 64 live columns of 128 counts as 64: its main loop skips the dead half); with fewer tiles the rounds they save
 // matter more (the h = 320 down dgrad ran 53% faster on large tiles at 2048 tokens, 3% slower at 8192).
 template <int EPI>
-static bool pick_large_mgroup(int64_t tiles_large, int64_t ncols) {
-  const int f = env_force();
-  if (f) return f == 1;
-  const int64_t cus = cu_count();
+static bool large_mgroup_rule(int64_t tiles_large, int64_t ncols, int64_t cus) {
   if (tiles_large >= 2 * cus) {
     const int64_t bl = EPI == EPI_SWIGLU ? CfgL::BN / 2 : CfgL::BN, bs = EPI == EPI_SWIGLU ? CfgS::BN / 2 : CfgS::BN;
     int64_t padl = (ncols + bl - 1) / bl * bl;
@@ -1129,6 +1126,12 @@ static bool pick_large_mgroup(int64_t tiles_large, int64_t ncols) {
     if (padl * 10 > pads * 11) return false;
   }
   return tiles_large * 8 >= cus * 5;
+}
+
+template <int EPI>
+static bool pick_large_mgroup(int64_t tiles_large, int64_t ncols) {
+  if (const int f = env_force()) return f == 1;
+  return large_mgroup_rule<EPI>(tiles_large, ncols, cu_count());
 }
 
 // int8 weights (forward only): several small workgroups share a CU and hide each other's conversions, prologues and
@@ -1141,10 +1144,15 @@ static bool pick_large_mgroup(int64_t tiles_large, int64_t ncols) {
 // By the 16-bit line 28% (gate/up) and 35% (down) of the launches with K below 512 and 12% of the other gate/up ones ran
 // more than 3% slower than with small tiles below 16 slices and, for gate/up, 2 1/2 tiles per CU; by these lines 2, 1 and 5%.
 template <int EPI>
+static bool large_i8_rule(int64_t tiles_large, int64_t ncols, int64_t K, int64_t cus) {
+  const int eighths = EPI == EPI_SWIGLU ? (K >= 768 ? 7 : K >= 384 ? 18 : 24) : (K >= 512 ? 6 : 48);
+  return large_mgroup_rule<EPI>(tiles_large, ncols, cus) && tiles_large * 8 >= cus * eighths;
+}
+
+template <int EPI>
 static bool pick_large_i8(int64_t tiles_large, int64_t ncols, int64_t K) {
   if (const int f = env_force()) return f == 1;
-  const int eighths = EPI == EPI_SWIGLU ? (K >= 768 ? 7 : K >= 384 ? 18 : 24) : (K >= 512 ? 6 : 48);
-  return pick_large_mgroup<EPI>(tiles_large, ncols) && tiles_large * 8 >= cu_count() * eighths;
+  return large_i8_rule<EPI>(tiles_large, ncols, K, cu_count());
 }
 
 template <int MODE, bool A_MN, bool B_MN, int EPI, bool A_BLK = false, bool F16 = false>
@@ -1209,7 +1217,7 @@ static FewTile pick_few(int64_t M, int64_t E, int64_t ncols, int64_t K, bool int
   if (t32 * 4 <= cus * 5 || (!GU && K <= 1280 && rows_to(24) && t32 <= 3 * cus)) return FEW_32x128;
   if (!rows_to(int8 && GU ? 132 : 112)) return FEW_NONE;
   const int64_t tl = mgroup_tiles<CfgL, EPI>(M, E, ncols);
-  const bool large = int8 ? pick_large_i8<EPI>(tl, ncols, K) : pick_large_mgroup<EPI>(tl, ncols);
+  const bool large = int8 ? large_i8_rule<EPI>(tl, ncols, K, cus) : large_mgroup_rule<EPI>(tl, ncols, cus);
   const int64_t rounds = large ? (tiles(256, 256) + cus - 1) / cus : (tiles(128, 128) + 2 * cus - 1) / (2 * cus);
   const int64_t t64 = tiles(64, 256), t128 = tiles(128, 256), most = 7 * cus * rounds;  // (fifths)
   const bool fit64 = (large || t64 * 4 >= 3 * cus) && t64 * 5 <= most, fit128 = t128 >= cus && t128 * 5 <= most;

@@ -251,7 +251,8 @@ def moe_block(x, gate_w, gate_b, k, n_group, topk_group, scaling, wgu, wgu_s, wd
     wd_s = _w_scale(wd, wd_s, d)
     _need(sh_wgu, "shared gate/up", (1, d, 2 * sh), _BF16)
     _need(sh_wd, "shared down", (1, sh, d), _BF16)
-    _need(sh_count, "shared row count", (1,), _I32)
+    if sh_count is None or sh_count.dtype is not torch.int32 or sh_count.shape != (1,) or not sh_count.is_cuda:
+        _need(sh_count, "shared row count", (1,), _I32)  # raises (called for every block it costs 1 us of about 80)
     w_dt = L.dt(wgu)
     ws_bytes = L.lib().hmoe_moe_block_workspace_size(T, d, E, k, h, sh, w_dt)
     if ws_bytes == 0:
