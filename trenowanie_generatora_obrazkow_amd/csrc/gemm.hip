@@ -1188,7 +1188,7 @@ static int launch_few_tile(const GemmParams& p, int64_t ncols, hipStream_t s) {
 // 1 to 200 rows per expert, even and Zipf 0.6-1.2 routing, every tile against the persistent kernel in one process, the
 // weights of successive calls apart (read from HBM).  Over these 13600 launches the choice takes 0.84 (16-bit gate/up), 0.85
 // (16-bit down), 0.80 and 0.79 (int8) of the persistent kernel's time in the geometric mean (the best tile of each launch:
-// 0.80, 0.82, 0.77, 0.77), and more than 3% longer in 1.9, 1.3, 1.0 and 3.4% of them; lines by the mean row count alone, 0.85,
+// 0.80, 0.82, 0.77, 0.77), and more than 3% longer in 1.9, 1.3, 2.2 and 3.4% of them; lines by the mean row count alone, 0.85,
 // 0.90, 0.80 and 0.81, in 5.8, 11.1, 5.2 and 6.7%.
 // What decides is how many workgroups a CU gets, with one m-tile for each expert that evenly routed rows would hit:
 //   32 rows x 128 columns up to 5/4 of them per CU (the launch is then one chain of latencies, and small tiles share it out
